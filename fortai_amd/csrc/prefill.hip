@@ -14,6 +14,8 @@
 #include "fortai_hip_internal.h"
 #include "fortai_hip_kernels.h"
 
+#include <type_traits>
+
 namespace fortai_hip {
 
 namespace {
@@ -513,14 +515,36 @@ __global__ __launch_bounds__(256) void attention_prefill_exact_kernel(const floa
     }
 }
 
-// The same arithmetic and orders with fixed trip counts: 16 queries per
-// workgroup (rows past the prompt are zero and never stored), keys clamped
-// into the cache and masked through zero weights, K / V tiles loaded one
-// ahead into registers, and (FINITE, no exponent-31 half in this cache) each
-// product fl(a * f32(h)) taken straight from the fp16 half by v_fma_mix_f32.
-// A workgroup whose cache is flagged returns unless !FINITE, and the !FINITE
-// instance serves only flagged caches, so the two launches split the work.
-constexpr int kXQ = 16;  // queries per workgroup
+// The same arithmetic and orders for prompts whose scores of QB queries fit in
+// LDS.  One workgroup of eight waves per (block of QB queries, head,
+// sequence).  The sums are chains of separately rounded products, so the
+// kernel is bound by vector issue and by the LDS reads beside it, and needs
+// many waves to cover the chains' dependent adds: QB is small, so that
+// several workgroups share a CU, and each lane owns a few chains whose
+// operands it shares in registers.
+//   scores: a wave owns 32 keys; its lanes are KG key groups x QB queries
+//     with KPL keys each.  No two waves share a key, so a key slice (32 keys x
+//     32 dims) sits in a buffer of the wave's own and the waves meet no
+//     barrier: a wave's LDS operations are in order.
+//   softmax weights: one wave per query, lanes over keys; Z by one lane.
+//   P.V: a thread owns DPL dims of one query; values pass through LDS 16
+//     keys at a time, double buffered, one barrier per tile.
+// Rows past the prompt are zero and never stored; keys are clamped into the
+// cache and masked through zero weights.  FINITE (no exponent-31 half in this
+// cache): each product fl(a * f32(h)) straight from the fp16 half by
+// v_fma_mix_f32.
+// Measured (one layer, heads of 256, against one workgroup of 16 queries per
+// CU pair with a barrier per key tile up to 512 positions and the kernel
+// above past them): 8 heads, 77 positions 57 -> 23 us, 511: 157 -> 67 us,
+// 2000: 4,610 -> 589 us; 16 heads, 1024: 2,886 -> 338 us.  At 2000 positions
+// its 256 M vector instructions are ~280 us of issue at eight waves per SIMD.
+// 64-key wave tiles (more chains per lane, fewer waves busy) 629 us, 16
+// queries per workgroup 717 us.
+constexpr int kXWaves = 8;
+constexpr size_t kXMaxLds = 160 * 1024;  // LDS of a CU
+constexpr int kXTileKeys = 32;   // keys per wave tile (scores)
+constexpr int kXValueKeys = 16;  // keys per staged value tile
+constexpr int kXSliceDims = 32;  // dims of a staged key slice
 
 template <bool FINITE>
 __device__ __forceinline__ float times_half(uint32_t h2, bool hi, float a) {
@@ -528,156 +552,206 @@ __device__ __forceinline__ float times_half(uint32_t h2, bool hi, float a) {
     return a * gguf_half_to_real(static_cast<uint16_t>(hi ? h2 >> 16 : h2 & 0xffffu));
 }
 
-template <int HEAD, bool FINITE>
-__global__ __launch_bounds__(256, 2) void attention_prefill_exact16_kernel(const float *__restrict__ q,
-    const uint16_t *__restrict__ kcache, const uint16_t *__restrict__ vcache, const int *__restrict__ flags,
-    float *__restrict__ out, int T, int heads, int kv_heads, int max_context, int kcap) {
-    static_assert(HEAD % 64 == 0 && HEAD <= 256, "head 64, 128 or 256");
-    constexpr int kPieces = kXKeys * HEAD / 8 / 256;  // 16-byte tile pieces per thread
-    constexpr int kQS = 256 / HEAD;                   // P.V: query phases per dim
-    constexpr int kQPT = kXQ / kQS;                   // P.V: queries per thread
-    extern __shared__ __align__(16) unsigned char lds_raw[];
-    float *qs = reinterpret_cast<float *>(lds_raw);                   // [16][HEAD] normalized q
-    uint16_t *kv = reinterpret_cast<uint16_t *>(qs + kXQ * HEAD);      // K: [HEAD/8][kXKeys][8]; V: [kXKeys][HEAD]
-    float *sc = reinterpret_cast<float *>(kv + kXKeys * HEAD);          // [16][kcap] scores, then e, then weights
+// bytes of LDS before the scores: q and the waves' key slices, or the two value tiles
+template <int HEAD, int QB>
+constexpr int attention_exact_stage_bytes() {
+    constexpr int qk = QB * HEAD * 4 + kXWaves * kXTileKeys * kXSliceDims * 2, v = 2 * kXValueKeys * HEAD * 2;
+    return qk > v ? qk : v;
+}
+
+template <int HEAD, int QB, bool FINITE>
+__device__ __forceinline__ void attention_exact_block(unsigned char *lds_raw, const float *__restrict__ q,
+    const uint16_t *__restrict__ kbase, const uint16_t *__restrict__ vbase, float *__restrict__ out, int T, int heads,
+    int kv_heads, int h, int s, int q0, int kcap) {
+    static_assert(QB == 4 || QB == 8, "one query per wave in the softmax");
+    constexpr int KG = 64 / QB, KPL = kXTileKeys / KG;
+    constexpr int kSlices = HEAD / kXSliceDims;
+    constexpr int kThreads = kXWaves * 64;
+    float *qs = reinterpret_cast<float *>(lds_raw);  // [QB][HEAD] normalized q
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
-    const int h = static_cast<int>(blockIdx.y), s = static_cast<int>(blockIdx.z);
-    const int kvh = h / (heads / kv_heads);
-    if ((flags[static_cast<size_t>(s) * kv_heads + kvh] != 0) == FINITE) return;
-    const int q0 = static_cast<int>(blockIdx.x) * kXQ;
-    const int nq = min(kXQ, T - q0);
-    const int keys = q0 + nq;                                       // keys 0..keys-1 cover the block
-    const int tiles = (keys + kXKeys - 1) / kXKeys, kpad = tiles * kXKeys;
+    uint4 *kb = reinterpret_cast<uint4 *>(lds_raw + QB * HEAD * 4) + wave * (kXTileKeys * kXSliceDims / 8);
+    uint16_t *vt = reinterpret_cast<uint16_t *>(lds_raw);  // [2][16][HEAD], after the scores
+    float *sc = reinterpret_cast<float *>(lds_raw + attention_exact_stage_bytes<HEAD, QB>());  // [QB][kcap]
+    const int nq = min(QB, T - q0);
+    const int keys = q0 + nq;  // keys 0..keys-1 cover the block
+    const int tiles = (keys + kXTileKeys - 1) / kXTileKeys, kpad = tiles * kXTileKeys;
     const float sqrt_head = sqrtf(static_cast<float>(HEAD));
-    const uint16_t *kbase = kcache + (static_cast<size_t>(s) * max_context * kv_heads + kvh) * HEAD;
-    const uint16_t *vbase = vcache + (static_cast<size_t>(s) * max_context * kv_heads + kvh) * HEAD;
     const size_t kvstride = static_cast<size_t>(kv_heads) * HEAD;
-    u32x4_t tile[kPieces];  // plain vectors (an array of the uint4 class would live in scratch)
-    // K tile piece e: key e / (HEAD/8), 8 dims (e % (HEAD/8)) of it; V tile piece e: the same key and dims
-    auto fetch = [&](const uint16_t *base, int j0) {
+
+    // ---- scores
+    // key slice piece (lane, n): key lane / 4 + 16 n, dims 8 (lane % 4) .. of the slice; stored at
+    // [piece][key ^ 2 piece], so neither the stores nor the reads of 8 consecutive keys meet a bank twice
+    u32x4_t kr[2];
+    const int pk = lane >> 2, pp = lane & 3;
+    auto fetch_k = [&](int t, int sl) {
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i) {
-            const int e = tid + 256 * i, j = e / (HEAD / 8), piece = e % (HEAD / 8);
-            tile[i] = *reinterpret_cast<const u32x4_t *>(base + static_cast<size_t>(min(j0 + j, keys - 1)) * kvstride +
-                piece * 8);
+        for (int n = 0; n < 2; ++n)
+            kr[n] = *reinterpret_cast<const u32x4_t *>(kbase +
+                static_cast<size_t>(min(t * kXTileKeys + pk + 16 * n, keys - 1)) * kvstride + sl * kXSliceDims + pp * 8);
+    };
+    if (wave < tiles) fetch_k(wave, 0);
+    for (int e = tid; e < QB * HEAD / 4; e += kThreads) {
+        const int qi = e / (HEAD / 4), d = e % (HEAD / 4);
+        float4 v = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (qi < nq)
+            v = reinterpret_cast<const float4 *>(q + ((static_cast<size_t>(s) * T + q0 + qi) * heads + h) * 2 * HEAD)[d];
+        reinterpret_cast<float4 *>(qs)[e] = v;
+    }
+    __syncthreads();
+    const int kg = lane % KG, qg = lane / KG;
+    for (int t = wave; t < tiles; t += kXWaves) {
+        float acc[KPL];
+#pragma unroll
+        for (int i = 0; i < KPL; ++i) acc[i] = 0.0f;
+#pragma unroll 1
+        for (int sl = 0; sl < kSlices; ++sl) {
+#pragma unroll
+            for (int n = 0; n < 2; ++n) {
+                const int key = pk + 16 * n;
+                *reinterpret_cast<u32x4_t *>(&kb[pp * kXTileKeys + (key ^ (2 * pp))]) = kr[n];
+            }
+            wave_lds_fence();
+            // the next slice (the last fetch of the wave is not used)
+            const bool wrap = sl + 1 == kSlices;
+            fetch_k(wrap ? min(t + kXWaves, tiles - 1) : t, wrap ? 0 : sl + 1);
+#pragma unroll
+            for (int pc = 0; pc < kXSliceDims / 8; ++pc) {
+                uint32_t kw[KPL][4];
+#pragma unroll
+                for (int i = 0; i < KPL; ++i) {
+                    const uint4 k8 = kb[pc * kXTileKeys + ((kg + KG * i) ^ (2 * pc))];
+                    kw[i][0] = k8.x; kw[i][1] = k8.y; kw[i][2] = k8.z; kw[i][3] = k8.w;
+                }
+                const float4 *qp = reinterpret_cast<const float4 *>(qs + qg * HEAD + sl * kXSliceDims + pc * 8);
+                const float4 qa = qp[0], qb = qp[1];
+                const float qv[8] = {qa.x, qa.y, qa.z, qa.w, qb.x, qb.y, qb.z, qb.w};
+                // the lane's chains interleaved (each chain's order unchanged)
+#pragma unroll
+                for (int k = 0; k < 8; ++k)
+#pragma unroll
+                    for (int i = 0; i < KPL; ++i)
+                        acc[i] = acc[i] + times_half<FINITE>(kw[i][k >> 1], (k & 1) != 0, qv[k]);
+            }
+            wave_lds_fence();
+        }
+#pragma unroll
+        for (int i = 0; i < KPL; ++i) sc[qg * kcap + t * kXTileKeys + kg + KG * i] = acc[i] / sqrt_head;
+    }
+    // the first value tile, while the weights are formed
+    constexpr int kVPieces = kXValueKeys * HEAD / 8;  // 16-byte pieces of a value tile
+    constexpr int kVLoads = (kVPieces + kThreads - 1) / kThreads;
+    u32x4_t vr[kVLoads];
+    auto fetch_v = [&](int t) {
+#pragma unroll
+        for (int n = 0; n < kVLoads; ++n) {
+            const int e = min(tid + kThreads * n, kVPieces - 1), j = e / (HEAD / 8), piece = e % (HEAD / 8);
+            vr[n] = *reinterpret_cast<const u32x4_t *>(vbase +
+                static_cast<size_t>(min(t * kXValueKeys + j, keys - 1)) * kvstride + piece * 8);
         }
     };
-    fetch(kbase, 0);
-    for (int e = tid; e < kXQ * HEAD; e += 256) {
-        const int qi = e / HEAD, d = e % HEAD;
-        qs[e] = qi < nq ? q[((static_cast<size_t>(s) * T + q0 + qi) * heads + h) * 2 * HEAD + d] : 0.0f;
-    }
-
-    // ---- scores: lane = key, wave = queries wave + 4 r
-    for (int t = 0; t < tiles; ++t) {
-        __syncthreads();  // the previous tile is consumed (and q is in place)
-#pragma unroll
-        for (int i = 0; i < kPieces; ++i) {
-            const int e = tid + 256 * i, j = e / (HEAD / 8), piece = e % (HEAD / 8);
-            *reinterpret_cast<u32x4_t *>(kv + (piece * kXKeys + j) * 8) = tile[i];
-        }
-        __syncthreads();
-        if (t + 1 < tiles) fetch(kbase, (t + 1) * kXKeys);
-        float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-        for (int d = 0; d < HEAD; d += 8) {
-            const uint4 k8 = *reinterpret_cast<const uint4 *>(kv + ((d / 8) * kXKeys + lane) * 8);
-            const uint32_t kw[4] = {k8.x, k8.y, k8.z, k8.w};
-            float qv[4][8];
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const float4 qa = *reinterpret_cast<const float4 *>(qs + (wave + 4 * r) * HEAD + d);
-                const float4 qc = *reinterpret_cast<const float4 *>(qs + (wave + 4 * r) * HEAD + d + 4);
-                qv[r][0] = qa.x; qv[r][1] = qa.y; qv[r][2] = qa.z; qv[r][3] = qa.w;
-                qv[r][4] = qc.x; qv[r][5] = qc.y; qv[r][6] = qc.z; qv[r][7] = qc.w;
-            }
-            // the four queries' chains interleaved (each chain's order unchanged),
-            // so consecutive adds do not wait on each other
-#pragma unroll
-            for (int k = 0; k < 8; ++k)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[r] = acc[r] + times_half<FINITE>(kw[k >> 1], (k & 1) != 0, qv[r][k]);
-        }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) sc[(wave + 4 * r) * kcap + t * kXKeys + lane] = acc[r] / sqrt_head;
-    }
-    fetch(vbase, 0);  // the first value tile, while the weights are formed
+    fetch_v(0);
     __syncthreads();
-    // ---- softmax weights: query wave + 4 r, lanes over keys; e = +0 past the query's keys
-    constexpr float kLowest = -3.402823466e38f;  // -huge(1.0_real32)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int qi = wave + 4 * r, n = min(q0 + qi + 1, keys);
-        float *row = sc + qi * kcap;
+    // ---- softmax weights of query `wave`: lanes over keys; e = +0 past the query's keys
+    if (wave < QB) {
+        constexpr float kLowest = -3.402823466e38f;  // -huge(1.0_real32)
+        const int n = min(q0 + wave + 1, keys);
+        float *row = sc + wave * kcap;
         float m = kLowest;
         for (int j = lane; j < n; j += 64) m = fmaxf(m, row[j]);
         m = wave_max(m);
         for (int j = lane; j < kpad; j += 64) row[j] = j < n ? expf_libm(row[j] - m) : 0.0f;
-    }
-    __syncthreads();
-    // Z of each query by one lane, left to right (the masked keys add +0)
-    if (lane < 4) {
-        const int qi = wave + 4 * lane;
-        const float *row = sc + qi * kcap;
+        wave_lds_fence();
+        // Z left to right (the masked keys add +0), by one lane: the reads of
+        // a whole wave would take the other waves' LDS bandwidth
+        const float4 *row4 = reinterpret_cast<const float4 *>(row);
         float z = 0.0f;
-        for (int j = 0; j < kpad; j += 4) {
-            const float4 e4 = *reinterpret_cast<const float4 *>(row + j);
-            z = z + e4.x;
-            z = z + e4.y;
-            z = z + e4.z;
-            z = z + e4.w;
-        }
-        qs[qi * HEAD] = z;  // q is no longer needed: slot 0 of the row holds Z
-    }
-    __syncthreads();
+        for (int j = 0; j < (lane == 0 ? kpad / 4 : 0); j += 8) {  // kpad % 32 == 0
+            float4 e4[8];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int qi = wave + 4 * r;
-        const float z = qs[qi * HEAD];
-        float *row = sc + qi * kcap;
+            for (int u = 0; u < 8; ++u) e4[u] = row4[j + u];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                z = z + e4[u].x;
+                z = z + e4[u].y;
+                z = z + e4[u].z;
+                z = z + e4[u].w;
+            }
+        }
+        wave_lds_fence();
+        z = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(z)));
         for (int j = lane; j < kpad; j += 64) row[j] = row[j] / z;
     }
 
-    // ---- P.V: thread = (dim d, queries qd + kQS r), keys left to right
-    const int d = tid % HEAD, qd = tid / HEAD;
-    float acc[kQPT];
+    // ---- P.V: thread = DPL dims of one query, keys left to right
+    const int vtiles = kpad / kXValueKeys;
+    constexpr int kCPT = QB * HEAD / kThreads;  // chains per thread
+    constexpr int DPL = kCPT >= 4 ? 4 : (kCPT >= 2 ? 2 : 1);
+    constexpr int LPQ = HEAD / DPL;  // threads per query
+    const int d0 = (tid % LPQ) * DPL, qi = tid / LPQ;
+    const float *wrow = sc + min(qi, QB - 1) * kcap;  // the narrowest blocks leave threads without a query
+    float acc[DPL];
 #pragma unroll
-    for (int r = 0; r < kQPT; ++r) acc[r] = 0.0f;
-    for (int t = 0; t < tiles; ++t) {
-        __syncthreads();  // the weights are complete / the previous tile is consumed
+    for (int d = 0; d < DPL; ++d) acc[d] = 0.0f;
+    for (int t = 0; t < vtiles; ++t) {
+        uint16_t *tile = vt + (t & 1) * kXValueKeys * HEAD;
 #pragma unroll
-        for (int i = 0; i < kPieces; ++i) {
-            const int e = tid + 256 * i, j = e / (HEAD / 8), piece = e % (HEAD / 8);
-            *reinterpret_cast<u32x4_t *>(kv + j * HEAD + piece * 8) = tile[i];
+        for (int n = 0; n < kVLoads; ++n) {
+            const int e = tid + kThreads * n;
+            if (kVPieces % kThreads == 0 || e < kVPieces) *reinterpret_cast<u32x4_t *>(tile + e * 8) = vr[n];
         }
+        // the tile is complete (and, the first time, the weights); the tile before last is consumed
         __syncthreads();
-        if (t + 1 < tiles) fetch(vbase, (t + 1) * kXKeys);
-        for (int jj = 0; jj < kXKeys; jj += 4) {
-            uint32_t vh[4];
+        if (t + 1 < vtiles) fetch_v(t + 1);
+#pragma unroll 2
+        for (int jj = 0; jj < kXValueKeys; jj += 4) {
+            uint32_t vh[4][DPL == 4 ? 2 : 1];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) vh[u] = kv[(jj + u) * HEAD + d];
-            float4 w4[kQPT];
+            for (int u = 0; u < 4; ++u) {
+                const uint16_t *vp = tile + (jj + u) * HEAD + d0;
+                if constexpr (DPL == 4) {
+                    const uint2 v2 = *reinterpret_cast<const uint2 *>(vp);
+                    vh[u][0] = v2.x; vh[u][1] = v2.y;
+                } else if constexpr (DPL == 2) {
+                    vh[u][0] = *reinterpret_cast<const uint32_t *>(vp);
+                } else {
+                    vh[u][0] = *vp;
+                }
+            }
+            const float4 w = *reinterpret_cast<const float4 *>(wrow + t * kXValueKeys + jj);
+            const float w4[4] = {w.x, w.y, w.z, w.w};
+            // the thread's chains interleaved key by key (each chain's order unchanged)
 #pragma unroll
-            for (int r = 0; r < kQPT; ++r)
-                w4[r] = *reinterpret_cast<const float4 *>(sc + (qd + kQS * r) * kcap + t * kXKeys + jj);
-            // the queries' chains interleaved key by key (each chain's order unchanged)
+            for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int r = 0; r < kQPT; ++r) acc[r] = acc[r] + times_half<FINITE>(vh[0], false, w4[r].x);
-#pragma unroll
-            for (int r = 0; r < kQPT; ++r) acc[r] = acc[r] + times_half<FINITE>(vh[1], false, w4[r].y);
-#pragma unroll
-            for (int r = 0; r < kQPT; ++r) acc[r] = acc[r] + times_half<FINITE>(vh[2], false, w4[r].z);
-#pragma unroll
-            for (int r = 0; r < kQPT; ++r) acc[r] = acc[r] + times_half<FINITE>(vh[3], false, w4[r].w);
+                for (int d = 0; d < DPL; ++d)
+                    acc[d] = acc[d] + times_half<FINITE>(vh[u][d >> 1], (d & 1) != 0, w4[u]);
         }
     }
+    if (qi >= nq) return;
+    const size_t row = (static_cast<size_t>(s) * T + q0 + qi) * heads + h;
 #pragma unroll
-    for (int r = 0; r < kQPT; ++r) {
-        const int qi = qd + kQS * r;
-        if (qi >= nq) continue;
-        const size_t row = (static_cast<size_t>(s) * T + q0 + qi) * heads + h;
-        const float gate = q[row * 2 * HEAD + HEAD + d];
-        out[row * HEAD + d] = acc[r] * sigmoid_ref(gate);
+    for (int d = 0; d < DPL; ++d) {
+        const float gate = q[row * 2 * HEAD + HEAD + d0 + d];
+        out[row * HEAD + d0 + d] = acc[d] * sigmoid_ref(gate);
     }
+}
+
+// blockIdx: x head, y sequence, z query block, the longest first (their keys
+// take the most time, so the last workgroups to start are the short ones)
+template <int HEAD, int QB>
+__global__ __launch_bounds__(kXWaves * 64, 4) void attention_prefill_exact_tiled_kernel(const float *__restrict__ q,
+    const uint16_t *__restrict__ kcache, const uint16_t *__restrict__ vcache, const int *__restrict__ flags,
+    float *__restrict__ out, int T, int heads, int kv_heads, int max_context, int kcap) {
+    static_assert(HEAD % 64 == 0 && HEAD <= 256, "head 64, 128 or 256");
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    const int h = static_cast<int>(blockIdx.x), s = static_cast<int>(blockIdx.y);
+    const int q0 = static_cast<int>(gridDim.z - 1 - blockIdx.z) * QB;
+    const int kvh = h / (heads / kv_heads);
+    const size_t first = (static_cast<size_t>(s) * max_context * kv_heads + kvh) * HEAD;
+    if (flags[static_cast<size_t>(s) * kv_heads + kvh] == 0)
+        attention_exact_block<HEAD, QB, true>(lds_raw, q, kcache + first, vcache + first, out, T, heads, kv_heads, h, s, q0, kcap);
+    else
+        attention_exact_block<HEAD, QB, false>(lds_raw, q, kcache + first, vcache + first, out, T, heads, kv_heads, h, s, q0, kcap);
 }
 
 // Causal attention of every prompt token (fortai_qwen35_cpu.f90:1006-1033
@@ -1105,37 +1179,42 @@ hipError_t launch_attention_prefill(const AttentionParams &p, int batch, int T, 
         if (e != hipSuccess) return e;
     }
     if (!matrix_cores) {
-        // 16 queries per workgroup when the block's scores fit in LDS (two
-        // launches: caches without and with exponent-31 halves)
-        const int kpad = (T + kXKeys - 1) / kXKeys * kXKeys;
-        const size_t lds16 = static_cast<size_t>(kXQ) * p.head * 4 + static_cast<size_t>(kXKeys) * p.head * 2 +
-            static_cast<size_t>(kXQ) * kpad * 4;
-        if (lds16 <= 80 * 1024) {
-            const dim3 xgrid((T + kXQ - 1) / kXQ, p.heads, batch);
-#define FORTAI_PREX(H)                                                                                              \
-    do {                                                                                                            \
-        hipLaunchKernelGGL((attention_prefill_exact16_kernel<H, true>), xgrid, dim3(256), lds16, stream, p.q,       \
-            p.kcache, p.vcache, p.cache_flags, out, T, p.heads, p.kv_heads, p.max_context, kpad);                   \
-        hipLaunchKernelGGL((attention_prefill_exact16_kernel<H, false>), xgrid, dim3(256), lds16, stream, p.q,      \
-            p.kcache, p.vcache, p.cache_flags, out, T, p.heads, p.kv_heads, p.max_context, kpad);                   \
-    } while (0)
-            switch (p.head) {
-            case 64: FORTAI_PREX(64); break;
-            case 128: FORTAI_PREX(128); break;
-            case 256: FORTAI_PREX(256); break;
-            default: return hipErrorInvalidValue;
-            }
-#undef FORTAI_PREX
-            note_launch("qk_rope_append_kernel grid %d + attention_prefill_exact16_kernel<%d> grid %dx%dx%d (x2)",
-                batch * T, p.head, xgrid.x, xgrid.y, xgrid.z);
+        // Four queries per workgroup while two workgroups fit on a CU (head
+        // 256: up to 3840 positions), eight while one fits (4352), four again
+        // (8960), then the kernel with global tiles and one to two queries.
+        // Head 256, 8 heads, QB 4 / 8: 511 positions 66 / 75 us, 2000: 586 /
+        // 807 us, 4100: 3,949 / 3,157 us.
+        const int kcap = (T + kXTileKeys - 1) / kXTileKeys * kXTileKeys;
+        int tiled = 0;
+        auto tiled_with = [&](auto qb_c, size_t lds_limit) {
+            constexpr int QB = decltype(qb_c)::value;
+            auto go = [&](auto head_c) {
+                constexpr int H = decltype(head_c)::value;
+                const size_t lds = static_cast<size_t>(attention_exact_stage_bytes<H, QB>()) + static_cast<size_t>(QB) * kcap * 4;
+                if (lds > lds_limit) return;
+                hipLaunchKernelGGL((attention_prefill_exact_tiled_kernel<H, QB>), dim3(p.heads, batch, (T + QB - 1) / QB),
+                    dim3(kXWaves * 64), lds, stream, p.q, p.kcache, p.vcache, p.cache_flags, out, T, p.heads, p.kv_heads,
+                    p.max_context, kcap);
+                tiled = QB;
+            };
+            if (p.head == 64) go(std::integral_constant<int, 64>{});
+            else if (p.head == 128) go(std::integral_constant<int, 128>{});
+            else go(std::integral_constant<int, 256>{});
+        };
+        tiled_with(std::integral_constant<int, 4>{}, kXMaxLds / 2);
+        if (!tiled) tiled_with(std::integral_constant<int, 8>{}, kXMaxLds);
+        if (!tiled) tiled_with(std::integral_constant<int, 4>{}, kXMaxLds);
+        if (tiled) {
+            note_launch("qk_rope_append_kernel grid %d + attention_prefill_exact_tiled_kernel<%d, %d> grid %dx%dx%d",
+                batch * T, p.head, tiled, p.heads, batch, (T + tiled - 1) / tiled);
             return hipGetLastError();
         }
         // longer prompts: queries per workgroup so that the block's scores fit in LDS
-        const int kcap = (T + 3) / 4 * 4;
-        int qb = 16;
+        const int kcap4 = (T + 3) / 4 * 4;
+        int qb = 4;
         auto lds_of = [&](int b) {
             return static_cast<size_t>(b) * p.head * 4 + static_cast<size_t>(kXKeys) * p.head * 2 +
-                static_cast<size_t>(b) * kcap * 4;
+                static_cast<size_t>(b) * kcap4 * 4;
         };
         while (qb > 1 && lds_of(qb) > 150 * 1024) qb /= 2;
         if (lds_of(qb) > 150 * 1024) return hipErrorInvalidValue;
@@ -1143,15 +1222,15 @@ hipError_t launch_attention_prefill(const AttentionParams &p, int batch, int T, 
         switch (p.head) {
         case 64:
             hipLaunchKernelGGL(attention_prefill_exact_kernel<64>, xgrid, dim3(256), lds_of(qb), stream, p.q, p.kcache,
-                p.vcache, out, T, p.heads, p.kv_heads, p.max_context, qb, kcap);
+                p.vcache, out, T, p.heads, p.kv_heads, p.max_context, qb, kcap4);
             break;
         case 128:
             hipLaunchKernelGGL(attention_prefill_exact_kernel<128>, xgrid, dim3(256), lds_of(qb), stream, p.q, p.kcache,
-                p.vcache, out, T, p.heads, p.kv_heads, p.max_context, qb, kcap);
+                p.vcache, out, T, p.heads, p.kv_heads, p.max_context, qb, kcap4);
             break;
         case 256:
             hipLaunchKernelGGL(attention_prefill_exact_kernel<256>, xgrid, dim3(256), lds_of(qb), stream, p.q, p.kcache,
-                p.vcache, out, T, p.heads, p.kv_heads, p.max_context, qb, kcap);
+                p.vcache, out, T, p.heads, p.kv_heads, p.max_context, qb, kcap4);
             break;
         default: return hipErrorInvalidValue;
         }

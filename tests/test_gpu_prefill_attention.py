@@ -112,3 +112,46 @@ def test_prefill_attention_kernels(ctx, oracle, head, T, big):
         A.free()
         for w in ws:
             w.free()
+
+
+@pytest.mark.parametrize("head,heads,kvh,T,big", [
+    (256, 4, 1, 3, False), (256, 4, 1, 31, False), (64, 4, 2, 33, False), (128, 8, 2, 65, True),
+    (256, 4, 1, 1029, False), (256, 2, 1, 545, True),
+    # the query-block rule's lines at head 64: 4 queries per workgroup to 4032
+    # positions, 8 to 4544, then 4 again
+    (64, 1, 1, 4032, False), (64, 1, 1, 4035, False), (64, 1, 1, 4545, False)])
+def test_exact_prefill_attention_blocks(ctx, oracle, head, heads, kvh, T, big):
+    """The tiled exact kernel at the edges of its key tiles, query blocks and
+    scores-in-LDS rule, bit for bit against the reference step (the appended
+    caches are checked above)."""
+    rng = np.random.default_rng(head * 7 + T)
+    rope = 16 if head == 64 else 64
+    mk = lambda rows, width: B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    ws = [mk(heads * 2 * head, 32), mk(kvh * head, 32), mk(kvh * head, 32), mk(32, heads * head)]
+    qn = (1 + 0.05 * rng.standard_normal(head)).astype(np.float32)
+    kn = (1 + 0.05 * rng.standard_normal(head)).astype(np.float32)
+    A = B.Attention(ctx, *ws, qn, kn, heads, kvh, head, head, T, rope, 1.0e7, 1e-6)
+    q = rng.standard_normal((T, heads * 2 * head)).astype(np.float32)
+    k = rng.standard_normal((T, kvh * head)).astype(np.float32)
+    v = rng.standard_normal((T, kvh * head)).astype(np.float32)
+    if big:
+        v[::5, : head // 2] *= np.float32(3e5)  # exponent-31 halves in kv head 0
+    kc, vc = np.zeros(T * kvh * head, np.uint16), np.zeros(T * kvh * head, np.uint16)
+    scores, want = np.zeros(T, np.float32), np.zeros((T, heads * head), np.float32)
+    for t in range(T):
+        qw, kw = q[t].copy(), k[t].copy()
+        oracle.attention_core_step(qw, kw, v[t].copy(), qn, kn, kc, vc, heads, kvh, head, head, t, rope,
+                                   np.float32(1e7), np.float32(1e-6), scores, want[t])
+    bufs = [ctx.upload_array(a) for a in (q, k, v)] + [ctx.alloc(T * heads * head * 4)]
+    try:
+        ctx.call("fortai_hip_qwen35_attention_prefill_core_device", A.h, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, T, 0,
+                 bufs[3].ptr)
+        got = bufs[3].download(np.float32).reshape(T, heads * head)
+        diff = [t for t in range(T) if not same_values(got[t], want[t])]
+        assert not diff, f"exact prefill attention differs from the reference step at rows {diff[:8]}"
+    finally:
+        for b in bufs:
+            b.free()
+        A.free()
+        for w in ws:
+            w.free()
