@@ -176,7 +176,7 @@ struct fortai_hip_qwen35_batch {
     const fortai_hip_f16_weights *emb16 = nullptr, *out16 = nullptr;
     const fortai_hip_q8_weights *emb8 = nullptr, *out8 = nullptr;
     float *output_norm = nullptr, *x = nullptr, *logits = nullptr;
-    float *xnorm = nullptr;  // output-RMSNormed x [hidden][8 slots], the fp16 LM head input
+    float *xnorm = nullptr;  // output-RMSNormed x [8 slots][hidden], the fp16 LM head input
     void *act = nullptr;     // quantized activations [batch][q8l_bytes(act_width)]
     void *h_q8l = nullptr;   // quantized FFN hidden [batch][q8l_bytes(ffn)]
     float *argmax_value = nullptr;

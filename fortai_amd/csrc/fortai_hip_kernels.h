@@ -150,7 +150,7 @@ hipError_t launch_f16_matvec(const uint16_t *w, int rows, int width, bool finite
     const float *norm, float eps, float *out, const ArgmaxState *argmax, hipStream_t stream);
 int f16_matvec_workgroups(int rows);
 // The fp16 LM head for `batch` (<= 8) sequences at once: final RMSNorm
-// (norm required) of x [batch][width] into xnorm [width][8] (interleaved), then
+// (norm required) of x [batch][width] into xnorm [8][width], then
 // out [batch][rows], argmax partials [batch][f16_batch_lm_head_workgroups(rows)]
 // and the per-sequence finish.
 hipError_t launch_f16_batch_lm_head(const uint16_t *w, int rows, int width, bool finite, int batch, const float *x,

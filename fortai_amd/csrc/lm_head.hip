@@ -18,6 +18,8 @@
 #include "fortai_hip_internal.h"
 #include "fortai_hip_kernels.h"
 
+#include <type_traits>
+
 namespace fortai_hip {
 
 namespace {
@@ -70,8 +72,22 @@ __global__ __launch_bounds__(256) void argmax_finish_kernel(int partials, Argmax
     if (st.embed && *st.embed >= 0) return;  // already finished (uniform)
     float bv = -__builtin_inff();
     int bi = 0x7fffffff;
-    for (int w = tid; w < partials; w += 256)
-        if (better(st.partial_value[w], st.partial_index[w], bv, bi)) { bv = st.partial_value[w]; bi = st.partial_index[w]; }
+    // kHeld * 256 partials per round trip (clamped; duplicates of the last
+    // partial change no first maximum): 3880 partials 7.6 -> 4.0 us
+    constexpr int kHeld = 8;
+    for (int w0 = tid; w0 < partials; w0 += kHeld * 256) {
+        float pv[kHeld];
+        int pi[kHeld];
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k) {
+            const int w = min(w0 + k * 256, partials - 1);
+            pv[k] = st.partial_value[w];
+            pi[k] = st.partial_index[w];
+        }
+#pragma unroll
+        for (int k = 0; k < kHeld; ++k)
+            if (better(pv[k], pi[k], bv, bi)) { bv = pv[k]; bi = pi[k]; }
+    }
     block_argmax(bv, bi, sv, si);
     if (tid == 0) {
         // no candidate (every logit NaN): the first index, as maxloc over
@@ -280,24 +296,20 @@ __global__ __launch_bounds__(kRows) void f16_matvec_kernel(const uint16_t *__res
     }
 }
 
-// Batched LM head: the fp16 table is read once for `batch` sequences.  Each
-// thread owns one row and runs, for every sequence, the same sequential chain
-// as f16_matvec_kernel (same tile order, same mul-then-add), and the final
-// RMSNorm of each sequence uses that kernel's reduction layout (128 strided
-// partial sums, then the two wave sums in order), so each sequence's logits
-// equal the single-sequence kernel's bit for bit.  256 rows x 64 columns per
-// tile; x of every sequence through scalar loads; per-sequence argmax partials.
-constexpr int kBatchRows = 256;
-constexpr int kBatchTile = 64;
-constexpr int kXCols = 8;  // columns of x per scalar-load batch in the batched LM head
+// Batched LM head: the fp16 table is read once for `batch` sequences.  A
+// workgroup takes 64 rows; wave s runs sequence s's sequential chain of every
+// row, one row per lane, with f16_matvec_kernel's order (product, then add),
+// and the final RMSNorm of each sequence uses that kernel's reduction layout
+// (128 strided partial sums, then the two wave sums in order), so each
+// sequence's logits equal the single-sequence kernel's bit for bit.
+constexpr int kBatchRows = 64;
 constexpr int kMaxBatch = 8;
 
 // Final RMSNorm of each sequence (fortai_qwen35_cpu.f90:707), one workgroup
 // of 128 threads per sequence with the single-sequence LM head's partition of
 // the sum (128 strided partial sums in double, the two wave sums in order), so
-// xnorm equals the x that kernel multiplies, bit for bit.  xnorm is
-// interleaved, [width][kMaxBatch]: workgroup s writes slot s with sequence
-// min(s, batch - 1), so the slots past the batch repeat the last sequence.
+// xnorm [slot][width] equals the x that kernel multiplies, bit for bit.  Slots
+// past the batch repeat the last sequence.
 __global__ __launch_bounds__(128) void batch_output_norm_kernel(const float *__restrict__ x,
     const float *__restrict__ norm, float eps, int width, int batch, float *__restrict__ xnorm) {
     FORTAI_TRACE_SCOPE(14);
@@ -316,125 +328,102 @@ __global__ __launch_bounds__(128) void batch_output_norm_kernel(const float *__r
     total += red[1];
     const float inv = 1.0f / sqrtf(static_cast<float>(div_count(total, width)) + eps);
 #pragma unroll 8
-    for (int i = tid; i < width; i += 128) xnorm[static_cast<size_t>(i) * kMaxBatch + slot] = (x[base + i] * inv) * norm[i];
+    for (int i = tid; i < width; i += 128) xnorm[static_cast<size_t>(slot) * width + i] = (x[base + i] * inv) * norm[i];
 }
 
-// xn: the normalized x of every sequence slot, interleaved [width][kMaxBatch].
-// Its addresses are uniform across the workgroup, so the 32 values of four
-// columns arrive by scalar loads into SGPRs and feed the VALU as operands: no
-// LDS traffic and no VGPRs for x (which would otherwise hold 64 floats per
-// column group and cap the occupancy at one wave per SIMD).
-template <bool FINITE>
-__global__ __launch_bounds__(kBatchRows) void f16_batch_lm_head_kernel(const uint16_t *__restrict__ w, int rows,
-    int width, int batch, const float *__restrict__ xn, float *__restrict__ out, ArgmaxState st) {
-    constexpr int kPitch = kBatchTile + 8;
-    extern __shared__ __align__(16) unsigned char lds[];
-    uint16_t *tile = reinterpret_cast<uint16_t *>(lds);
-    __shared__ float sv[kBatchRows / 64];
-    __shared__ int si[kBatchRows / 64];
-    const int tid = static_cast<int>(threadIdx.x);
+// NW waves (the batch rounded up to a power of two; slots past it repeat the
+// last sequence and are not written).  xn: the normalized x [slot][width]; a
+// wave's x addresses are uniform, so x arrives by scalar loads and feeds the
+// vector operations from SGPRs.  One sequence per wave keeps a lane at a
+// single chain and few registers (eight waves per SIMD cover each other's
+// waits) and gives a small table enough waves: with 256 rows per workgroup and
+// eight chains per lane, a 16384 x 2560 table ran in 64 workgroups, 170 us
+// (now 48), and a batch below eight paid for all eight chains (248320 x 2560:
+// batch 8 330 -> 317 us, batch 1 330 -> 189 us).
+template <bool FINITE, int NW, int TILE>
+__global__ __launch_bounds__(64 * NW) void f16_batch_lm_head_kernel(const uint16_t *__restrict__ w, int rows, int width,
+    int batch, const float *__restrict__ xn, float *__restrict__ out, ArgmaxState st) {
+    constexpr int kPitch = TILE + 8;
+    constexpr int kThreads = 64 * NW;
+    __shared__ __align__(16) uint16_t tile[kBatchRows * kPitch];
+    const int tid = static_cast<int>(threadIdx.x), lane = tid & 63;
+    const int seq = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int row0 = static_cast<int>(blockIdx.x) * kBatchRows;
 
-    constexpr int kSegs = kBatchTile / 8;
-    constexpr int kLoads = kBatchTile * 2 / 16;  // 16-byte loads per thread and tile (one row's worth)
+    constexpr int kSegs = TILE / 8;
+    constexpr int kLoads = kBatchRows * kSegs / kThreads;  // 16-byte loads per thread and tile
     uint4 ra[kLoads], rb[kLoads];
     auto fetch = [&](int k0, uint4 (&regs)[kLoads]) {
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) {
-            const int li = tid + kBatchRows * j;
+            const int li = tid + kThreads * j;
             const int r = li / kSegs, seg = li % kSegs;
-            const int grow = min(row0 + r, rows - 1);
+            const int grow = min(row0 + r, rows - 1);  // rows past the end re-read the last row
             regs[j] = load_stream(reinterpret_cast<const uint4 *>(w + static_cast<size_t>(grow) * width + k0 + seg * 8));
         }
     };
     auto stash = [&](const uint4 (&regs)[kLoads]) {
 #pragma unroll
         for (int j = 0; j < kLoads; ++j) {
-            const int li = tid + kBatchRows * j;
+            const int li = tid + kThreads * j;
             const int r = li / kSegs, seg = li % kSegs;
             *reinterpret_cast<uint4 *>(tile + r * kPitch + seg * 8) = regs[j];
         }
     };
-    const int tiles = width / kBatchTile;
+    const int tiles = width / TILE;
     fetch(0, ra);
-    if (tiles > 1) fetch(kBatchTile, rb);
-
-    // every sequence slot is computed (slots past the batch repeat the last
-    // sequence and are not written): no per-sequence branch in the inner loop
-    float acc[kMaxBatch];
-#pragma unroll
-    for (int s = 0; s < kMaxBatch; ++s) acc[s] = 0.0f;
-    // kXCols columns per scalar-load round trip (8 x kXCols SGPRs of x; the
-    // wait for them is a full lgkmcnt(0), so more columns per load means
-    // fewer exposed waits; the other waves of the SIMD cover the rest)
-    auto xload = [&](int k, float (&xv)[kXCols][kMaxBatch]) {
-        const float4 *src = reinterpret_cast<const float4 *>(xn + static_cast<size_t>(k) * kMaxBatch);
-#pragma unroll
-        for (int i = 0; i < kXCols * kMaxBatch / 4; ++i) {
-            const float4 v = src[i];
-            xv[i / 2][(i % 2) * 4 + 0] = v.x;
-            xv[i / 2][(i % 2) * 4 + 1] = v.y;
-            xv[i / 2][(i % 2) * 4 + 2] = v.z;
-            xv[i / 2][(i % 2) * 4 + 3] = v.w;
-        }
-    };
-    auto step = [&](const uint16_t *mine, int c, const float (&xv)[kXCols][kMaxBatch], int x0) {
-        const uint2 h4 = *reinterpret_cast<const uint2 *>(mine + c * 4);
-        float a[4];
-        a[0] = FINITE ? half_bits_to_float(static_cast<uint16_t>(h4.x & 0xffffu))
-                      : gguf_half_to_real(static_cast<uint16_t>(h4.x & 0xffffu));
-        a[1] = FINITE ? half_bits_to_float(static_cast<uint16_t>(h4.x >> 16))
-                      : gguf_half_to_real(static_cast<uint16_t>(h4.x >> 16));
-        a[2] = FINITE ? half_bits_to_float(static_cast<uint16_t>(h4.y & 0xffffu))
-                      : gguf_half_to_real(static_cast<uint16_t>(h4.y & 0xffffu));
-        a[3] = FINITE ? half_bits_to_float(static_cast<uint16_t>(h4.y >> 16))
-                      : gguf_half_to_real(static_cast<uint16_t>(h4.y >> 16));
-#pragma unroll
-        for (int s = 0; s < kMaxBatch; ++s) {
-            float v = acc[s];
-            v = v + a[0] * xv[x0][s]; v = v + a[1] * xv[x0 + 1][s]; v = v + a[2] * xv[x0 + 2][s];
-            v = v + a[3] * xv[x0 + 3][s];
-            acc[s] = v;
-        }
-    };
+    fetch(min(TILE, width - TILE), rb);  // (one tile: a harmless second copy)
+    const float *x = xn + static_cast<size_t>(seq) * width;
+    float acc = 0.0f;
     auto consume = [&](int k0) {
-        const uint16_t *mine = tile + tid * kPitch;
-#pragma unroll 1
-        for (int c = 0; c < kBatchTile / 4; c += kXCols / 4) {
-            float xv[kXCols][kMaxBatch];
-            xload(k0 + c * 4, xv);
+        const uint16_t *mine = tile + lane * kPitch;
 #pragma unroll
-            for (int u = 0; u < kXCols / 4; ++u) step(mine, c + u, xv, 4 * u);
+        for (int s = 0; s < kSegs; ++s) {
+            const uint4 h8 = *reinterpret_cast<const uint4 *>(mine + s * 8);
+            const uint32_t hw[4] = {h8.x, h8.y, h8.z, h8.w};
+            float p[8];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float x0 = x[k0 + s * 8 + 2 * q], x1 = x[k0 + s * 8 + 2 * q + 1];
+                if constexpr (FINITE) {
+                    p[2 * q] = half_times<false>(hw[q], x0);
+                    p[2 * q + 1] = half_times<true>(hw[q], x1);
+                } else {
+                    p[2 * q] = gguf_half_to_real(static_cast<uint16_t>(hw[q] & 0xffffu)) * x0;
+                    p[2 * q + 1] = gguf_half_to_real(static_cast<uint16_t>(hw[q] >> 16)) * x1;
+                }
+            }
+#pragma unroll
+            for (int q = 0; q < 8; ++q) acc = acc + p[q];
         }
     };
     for (int t = 0; t < tiles; t += 2) {
         __syncthreads();
         stash(ra);
         __syncthreads();
-        if (t + 2 < tiles) fetch((t + 2) * kBatchTile, ra);
-        consume(t * kBatchTile);
+        if (t + 2 < tiles) fetch((t + 2) * TILE, ra);
+        consume(t * TILE);
         if (t + 1 >= tiles) break;
         __syncthreads();
         stash(rb);
         __syncthreads();
-        if (t + 3 < tiles) fetch((t + 3) * kBatchTile, rb);
-        consume((t + 1) * kBatchTile);
+        if (t + 3 < tiles) fetch((t + 3) * TILE, rb);
+        consume((t + 1) * TILE);
     }
-    const int row = row0 + tid;
-    const int parts = static_cast<int>(gridDim.x);
-#pragma unroll
-    for (int s = 0; s < kMaxBatch; ++s) {
-        if (s < batch) {
-            if (row < rows) out[static_cast<size_t>(s) * rows + row] = acc[s];
-            float v = row < rows ? acc[s] : -__builtin_inff();
-            int i = row < rows ? row : 0x7fffffff;
-            block_argmax(v, i, sv, si);
-            if (tid == 0) {
-                st.partial_value[static_cast<size_t>(s) * parts + blockIdx.x] = v;
-                st.partial_index[static_cast<size_t>(s) * parts + blockIdx.x] = i;
-            }
-            __syncthreads();  // sv / si are reused by the next sequence
-        }
+    if (seq >= batch) return;
+    const int row = row0 + lane;
+    if (row < rows) out[static_cast<size_t>(seq) * rows + row] = acc;
+    float v = row < rows ? acc : -__builtin_inff();
+    int i = row < rows ? row : 0x7fffffff;
+    argmax_step<32>(v, i);
+    argmax_step<16>(v, i);
+    argmax_step<8>(v, i);
+    argmax_step<4>(v, i);
+    argmax_step<2>(v, i);
+    argmax_step<1>(v, i);
+    if (lane == 0) {
+        st.partial_value[static_cast<size_t>(seq) * gridDim.x + blockIdx.x] = v;
+        st.partial_index[static_cast<size_t>(seq) * gridDim.x + blockIdx.x] = i;
     }
 }
 
@@ -508,25 +497,36 @@ int f16_batch_lm_head_workgroups(int rows) { return (rows + kBatchRows - 1) / kB
 
 hipError_t launch_f16_batch_lm_head(const uint16_t *w, int rows, int width, bool finite, int batch, const float *x,
     const float *norm, float eps, float *xnorm, float *out, const ArgmaxState &argmax, hipStream_t stream) {
-    if (rows <= 0 || width <= 0 || width % kBatchTile || batch < 1 || batch > kMaxBatch || !norm || !xnorm)
+    if (rows <= 0 || width <= 0 || width % 64 || batch < 1 || batch > kMaxBatch || !norm || !xnorm)
         return hipErrorInvalidValue;
     const int grid = f16_batch_lm_head_workgroups(rows);
-    hipLaunchKernelGGL(batch_output_norm_kernel, dim3(kMaxBatch), dim3(128), 0, stream, x, norm, eps, width, batch,
-        xnorm);
+    const int waves = batch <= 2 ? batch : (batch <= 4 ? 4 : 8);
+    hipLaunchKernelGGL(batch_output_norm_kernel, dim3(waves), dim3(128), 0, stream, x, norm, eps, width, batch, xnorm);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const size_t lds = static_cast<size_t>(kBatchRows) * (kBatchTile + 8) * 2;
-    if (finite)
-        hipLaunchKernelGGL(f16_batch_lm_head_kernel<true>, dim3(grid), dim3(kBatchRows), lds, stream, w, rows, width,
-            batch, xnorm, out, argmax);
-    else
-        hipLaunchKernelGGL(f16_batch_lm_head_kernel<false>, dim3(grid), dim3(kBatchRows), lds, stream, w, rows, width,
-            batch, xnorm, out, argmax);
+    auto go = [&](auto finite_c, auto waves_c) {
+        constexpr bool F = decltype(finite_c)::value;
+        constexpr int NW = decltype(waves_c)::value;
+        if (width % 128 == 0)  // 128-column tiles where the width allows, else 64
+            hipLaunchKernelGGL((f16_batch_lm_head_kernel<F, NW, 128>), dim3(grid), dim3(64 * NW), 0, stream, w, rows, width,
+                batch, xnorm, out, argmax);
+        else
+            hipLaunchKernelGGL((f16_batch_lm_head_kernel<F, NW, 64>), dim3(grid), dim3(64 * NW), 0, stream, w, rows, width,
+                batch, xnorm, out, argmax);
+    };
+    auto pick = [&](auto finite_c) {
+        if (waves == 1) go(finite_c, std::integral_constant<int, 1>{});
+        else if (waves == 2) go(finite_c, std::integral_constant<int, 2>{});
+        else if (waves == 4) go(finite_c, std::integral_constant<int, 4>{});
+        else go(finite_c, std::integral_constant<int, 8>{});
+    };
+    if (finite) pick(std::true_type{});
+    else pick(std::false_type{});
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     e = launch_argmax_finish(grid, argmax, stream, batch);
     note_launch("batch_output_norm_kernel grid %d + f16_batch_lm_head_kernel<finite=%d> grid %d + argmax_finish_kernel "
-        "grid 1x%d", kMaxBatch, finite, grid, batch);
+        "grid 1x%d", waves, finite, grid, batch);
     return e;
 }
 

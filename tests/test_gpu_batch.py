@@ -169,3 +169,25 @@ def test_batch_matvec_bit_identical(ctx, oracle, rows, width, batch):
         want = oracle.matvec(w, rows, width, x[s])
         assert np.array_equal(got[s].view(np.uint32), want.view(np.uint32)), f"row {s}"
     W.free()
+
+
+@pytest.mark.parametrize("batch", [1, 2, 4, 6])
+@pytest.mark.parametrize("hidden,vocab", [(320, 1000), (384, 65)])
+def test_batch_lm_head_shapes(tmp_path, hidden, vocab, batch):
+    """The batched fp16 LM head at 64- and 128-column tiles, ragged 64-row
+    workgroups and every wave count (1, 2, 4, 8): bits of the single-sequence
+    decoder's logits."""
+    from dataclasses import replace
+    path = str(tmp_path / "lm.gguf")
+    synth.write_model(path, replace(synth.CONFIGS["qwen35-tiny"], name="lm", hidden=hidden, vocab=vocab))
+    m = Qwen35Hip(path, max_context=16, batch=batch)
+    try:
+        tokens = np.arange(batch, dtype=np.int64) * 7 % vocab
+        m.batch.reset()
+        nxt = m.batch.forward(tokens, np.zeros(batch, dtype=np.int32))
+        for s in range(batch):
+            want_logits, want_tokens = run_single(m, int(tokens[s]), 0, 1)
+            assert np.array_equal(m.batch.logits[s].view(np.uint32), want_logits[0].view(np.uint32)), f"sequence {s}"
+            assert int(nxt[s]) == want_tokens[0]
+    finally:
+        m.close()
