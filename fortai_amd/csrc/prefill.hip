@@ -215,80 +215,156 @@ __global__ __launch_bounds__(256) void gdn_token_prep_kernel(const float *__rest
     }
 }
 
-// The delta rule over time (fortai_q8_dot.c:356-398) for 16 state rows of one
-// value head of one sequence (blockIdx.y), the state in registers in the
-// decode kernel's layout: S[row][8 i + l] at
-// state[((h * HEAD + row) * 8 + l) * HEAD/8 + i].  Normalized q and k of
-// kStage tokens are staged in LDS at a time.
-constexpr int kGdnRows = 16;
-constexpr int kStage = 16;
+// The delta rule over time (fortai_q8_dot.c:356-398), the state in registers
+// in the decode kernel's layout: S[row][8 i + l] at
+// state[((h * HEAD + row) * 8 + l) * HEAD/8 + i].  A one-wave workgroup runs
+// 8 rows of one value head of one sequence (blockIdx.y), lane l of a row its
+// eighth.  The steps are a serial chain, so what counts is the latency
+// of one: no barrier (the wave's own LDS operations are in order), nothing
+// waited for inside a step, and two chains in flight -- the q dot of token t
+// and the decay and k dot of token t + 1 run interleaved over the columns
+// (each chain in its own order).  Tokens reach LDS kGdnChunk at a time from
+// registers loaded one chunk ahead; a step's reads are issued before the
+// horizontal sum that its column loop waits for.  A lane's 16 columns are
+// contiguous with a 4-float pad per lane, so its 16-byte reads meet no bank
+// twice.
+// Measured (head 128, against 16 rows per two-wave workgroup with two barriers
+// per 16 tokens and four-byte reads): 16 heads x 77 tokens 59 -> 24 us, 32
+// heads x 3 x 701 538 -> 270 us, 32 heads x 8 x 512 490 -> 342 us.  Two rows per
+// lane (each read of q and k shared) 414 us at the last.
+constexpr int kGdnChunk = 4;
 
 template <int HEAD>
-__global__ __launch_bounds__(kGdnRows * 8) void gdn_prefill_kernel(const float *__restrict__ qkv,
+__global__ __launch_bounds__(64) void gdn_prefill_kernel(const float *__restrict__ qkv,
     const float *__restrict__ qinv, const float *__restrict__ kinv, const float *__restrict__ beta,
     const float *__restrict__ decay, float *__restrict__ state, float *__restrict__ out, int T, int C, int key_heads,
     int value_heads, int state_size) {
-    constexpr int kCols = HEAD / 8;
-    __shared__ __align__(16) float qs[kStage][HEAD];
-    __shared__ __align__(16) float ks[kStage][HEAD];
-    __shared__ float vs[kStage][kGdnRows];
-    __shared__ float bs[kStage], ds[kStage];
-    const int tid = static_cast<int>(threadIdx.x);
+    constexpr int kCols = HEAD / 8, kPitch = kCols + 4, kRows = 8;
+    constexpr int kSlot = 2 * 8 * kPitch;
+    // per token: q [8][kPitch], k [8][kPitch]; the 4-float pads of the 16 lane
+    // rows hold 64 aux words: v of the rows, then beta, decay (and copies of it)
+    __shared__ __align__(16) float ring[2 * kGdnChunk * kSlot];
+    auto aux = [](int i) { return (i >> 2) * kPitch + kCols + (i & 3); };
+    const int lane = static_cast<int>(threadIdx.x);
     const int s = static_cast<int>(blockIdx.y);
-    const int bph = HEAD / kGdnRows;
-    const int h = static_cast<int>(blockIdx.x) / bph, r0 = (static_cast<int>(blockIdx.x) % bph) * kGdnRows;
+    constexpr int kBlocks = HEAD / kRows;
+    const int h = static_cast<int>(blockIdx.x) / kBlocks, r0 = (static_cast<int>(blockIdx.x) % kBlocks) * kRows;
     const int kh = h / (value_heads / key_heads);
-    const int r8 = tid >> 3, l = tid & 7, row = r0 + r8;
+    const int r8 = lane >> 3, l = lane & 7;
     const int inner = value_heads * HEAD;
-    float *sp = state + static_cast<size_t>(s) * value_heads * HEAD * HEAD + ((static_cast<size_t>(h) * HEAD + row) * 8 + l) * kCols;
+    float *sp = state + static_cast<size_t>(s) * value_heads * HEAD * HEAD +
+        ((static_cast<size_t>(h) * HEAD + r0 + r8) * 8 + l) * kCols;
     float st[kCols];
 #pragma unroll
     for (int i = 0; i < kCols; ++i) st[i] = sp[i];
     const float scale = 1.0f / sqrtf(static_cast<float>(HEAD));
-    for (int t0 = 0; t0 < T; t0 += kStage) {
-        const int steps = min(kStage, T - t0);
-        __syncthreads();  // the previous stage is consumed
+    // this lane's share of a token: 4 values of q (lanes < HEAD/4) or k, the
+    // head's inverse norm, and one aux word
+    const bool has_qk = lane < HEAD / 2;
+    const int ql = has_qk ? lane : 0, isk = ql >= HEAD / 4, c4 = (ql % (HEAD / 4)) * 4;
+    const float *qk_src = qkv + (isk ? state_size * key_heads : 0) + kh * HEAD + c4;
+    const float *inv_src = (isk ? kinv : qinv) + kh;
+    const int al = min(lane, kRows + 1);
+    const float *aux_src = al < kRows ? qkv + 2 * state_size * key_heads + h * HEAD + r0 + al
+                                      : (al == kRows ? beta : decay) + h;
+    const int aux_pitch = al < kRows ? C : value_heads;
+    float4 fq[kGdnChunk];
+    float fi[kGdnChunk], fa[kGdnChunk];
+    auto fetch = [&](int chunk) {
 #pragma unroll
-        for (int e = tid; e < kStage * HEAD; e += kGdnRows * 8) {
-            const int j = e / HEAD, i = e % HEAD;
-            const size_t n = static_cast<size_t>(s) * T + t0 + min(j, steps - 1);
-            const float *rowp = qkv + n * C;
-            qs[j][i] = rowp[kh * HEAD + i] * qinv[n * key_heads + kh];
-            ks[j][i] = rowp[state_size * key_heads + kh * HEAD + i] * kinv[n * key_heads + kh];
+        for (int j = 0; j < kGdnChunk; ++j) {
+            const size_t n = static_cast<size_t>(s) * T + min(chunk * kGdnChunk + j, T - 1);
+            fq[j] = *reinterpret_cast<const float4 *>(qk_src + n * C);
+            fi[j] = inv_src[n * key_heads];
+            fa[j] = aux_src[n * aux_pitch];
         }
+    };
+    auto stash = [&](int chunk) {
+        float *base = ring + (chunk & 1) * (kGdnChunk * kSlot);
 #pragma unroll
-        for (int e = tid; e < kStage * kGdnRows; e += kGdnRows * 8) {
-            const int j = e / kGdnRows, rr = e % kGdnRows;
-            const size_t n = static_cast<size_t>(s) * T + t0 + min(j, steps - 1);
-            vs[j][rr] = qkv[n * C + 2 * state_size * key_heads + h * HEAD + r0 + rr];
-        }
-        if (tid < kStage) {
-            const size_t n = static_cast<size_t>(s) * T + t0 + min(tid, steps - 1);
-            bs[tid] = beta[n * value_heads + h];
-            ds[tid] = decay[n * value_heads + h];
-        }
-        __syncthreads();
-        for (int j = 0; j < steps; ++j) {
-            const float dec = ds[j];
-            float kd = 0.0f;
+        for (int j = 0; j < kGdnChunk; ++j) {
+            float *slot = base + j * kSlot;
+            const float v[4] = {fq[j].x, fq[j].y, fq[j].z, fq[j].w};
+            if (HEAD == 128 || has_qk) {
+                float *dst = slot + isk * 8 * kPitch + c4 / 8;
 #pragma unroll
-            for (int i = 0; i < kCols; ++i) {
-                const float d = st[i] * dec;
-                st[i] = d;
-                kd = __builtin_fmaf(d, ks[j][8 * i + l], kd);
+                for (int u = 0; u < 4; ++u) dst[((c4 & 4) + u) * kPitch] = v[u] * fi[j];
             }
-            kd = row_hsum8(kd);
-            const float delta = (vs[j][r8] - kd) * bs[j];
-            float qd = 0.0f;
-#pragma unroll
-            for (int i = 0; i < kCols; ++i) {
-                const float u = __builtin_fmaf(delta, ks[j][8 * i + l], st[i]);
-                st[i] = u;
-                qd = __builtin_fmaf(u, qs[j][8 * i + l], qd);
-            }
-            qd = row_hsum8(qd);
-            if (l == 0) out[(static_cast<size_t>(s) * T + t0 + j) * inner + h * HEAD + row] = qd * scale;
+            slot[aux(lane)] = fa[j];
         }
+        wave_lds_fence();
+    };
+    struct Token {  // k, v and beta of a token
+        float k[kCols], v, b;
+    };
+    auto read_cols = [&](const float *src, float (&dst)[kCols]) {
+#pragma unroll
+        for (int i = 0; i < kCols / 4; ++i) {
+            const float4 f = reinterpret_cast<const float4 *>(src + l * kPitch)[i];
+            dst[4 * i] = f.x; dst[4 * i + 1] = f.y; dst[4 * i + 2] = f.z; dst[4 * i + 3] = f.w;
+        }
+    };
+    auto read_token = [&](const float *slot, Token &t, float &d) {
+        read_cols(slot + 8 * kPitch, t.k);
+        t.v = slot[aux(r8)];
+        t.b = slot[aux(kRows)];
+        d = slot[aux(kRows + 1)];
+    };
+    fetch(0);
+    stash(0);
+    fetch(1);
+    Token ta, tb;
+    float kd = 0.0f;
+    {
+        float d0;
+        read_token(ring, ta, d0);
+#pragma unroll
+        for (int i = 0; i < kCols; ++i) {
+            const float d = st[i] * d0;
+            st[i] = d;
+            kd = __builtin_fmaf(d, ta.k[i], kd);
+        }
+    }
+    float *orow = out + static_cast<size_t>(s) * T * inner + h * HEAD + r0 + r8;
+    // token t (its slot) with token t + 1's decay and k dot
+    auto step = [&](int t, const float *slot, const float *slot1, const Token &cur, Token &nxt) {
+        float q[kCols], dn;
+        read_token(slot1, nxt, dn);
+        read_cols(slot, q);
+        __builtin_amdgcn_sched_barrier(0);
+        const float delta = (cur.v - row_hsum8(kd)) * cur.b;
+        if (t + 1 >= T) dn = 1.0f;  // past the last token the state is kept: a factor of one
+        float qd = 0.0f;
+        kd = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kCols; ++i) {
+            const float u = __builtin_fmaf(delta, cur.k[i], st[i]);
+            qd = __builtin_fmaf(u, q[i], qd);
+            const float d = u * dn;
+            st[i] = d;
+            kd = __builtin_fmaf(d, nxt.k[i], kd);
+        }
+        // every lane of the row stores the same value: a branch here would
+        // keep the compiler from interleaving the two chains
+        orow[static_cast<size_t>(t) * inner] = row_hsum8(qd) * scale;
+    };
+    static_assert(kGdnChunk == 4, "the two tokens' registers swap an even number of times per chunk");
+    int c = 0;
+    for (; (c + 1) * kGdnChunk <= T; ++c) {
+        const int t = c * kGdnChunk;
+        const float *here = ring + (c & 1) * (kGdnChunk * kSlot), *other = ring + ((c & 1) ^ 1) * (kGdnChunk * kSlot);
+        step(t, here, here + kSlot, ta, tb);
+        step(t + 1, here + kSlot, here + 2 * kSlot, tb, ta);
+        stash(c + 1);
+        fetch(c + 2);
+        step(t + 2, here + 2 * kSlot, here + 3 * kSlot, ta, tb);
+        step(t + 3, here + 3 * kSlot, other, tb, ta);
+    }
+    // the last, partial chunk (its slot past the end is read but not used)
+    const float *here = ring + (c & 1) * (kGdnChunk * kSlot);
+    for (int t = c * kGdnChunk; t < T; ++t, here += kSlot) {
+        step(t, here, here + kSlot, ta, tb);
+        ta = tb;
     }
 #pragma unroll
     for (int i = 0; i < kCols; ++i) sp[i] = st[i];
@@ -1124,18 +1200,14 @@ hipError_t launch_gdn_prefill(const GdnParams &p, int batch, int T, float *qinv,
         p.ssm_dt, C, p.key_heads, p.value_heads, p.head, p.state_size, p.eps, qinv, kinv, beta_t, decay_t);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
-    const dim3 grid(p.value_heads * (p.head / kGdnRows), batch);
-    switch (p.head) {
-    case 64:
-        hipLaunchKernelGGL(gdn_prefill_kernel<64>, grid, dim3(kGdnRows * 8), 0, stream, p.qkv, qinv, kinv, beta_t,
-            decay_t, p.state, p.out, T, C, p.key_heads, p.value_heads, p.state_size);
-        break;
-    case 128:
-        hipLaunchKernelGGL(gdn_prefill_kernel<128>, grid, dim3(kGdnRows * 8), 0, stream, p.qkv, qinv, kinv, beta_t,
-            decay_t, p.state, p.out, T, C, p.key_heads, p.value_heads, p.state_size);
-        break;
-    default: return hipErrorInvalidValue;
-    }
+    const dim3 grid(p.value_heads * (p.head / 8), batch);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(64), 0, stream, p.qkv, qinv, kinv, beta_t, decay_t, p.state, p.out, T, C,
+            p.key_heads, p.value_heads, p.state_size);
+    };
+    if (p.head == 64) go(gdn_prefill_kernel<64>);
+    else if (p.head == 128) go(gdn_prefill_kernel<128>);
+    else return hipErrorInvalidValue;
     note_launch("gdn_token_prep_kernel grid %d + gdn_prefill_kernel<%d> grid %dx%d", rows, p.head, grid.x, batch);
     return hipGetLastError();
 }

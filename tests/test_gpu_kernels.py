@@ -401,3 +401,35 @@ def test_f16_lm_head_and_argmax(ctx, oracle):
     ctx.call("fortai_hip_argmax_device", ctx.h, dn.ptr, 100000, dt.ptr)
     assert int(dt.download(np.int64)[0]) == 0
     W.free()
+
+
+@pytest.mark.parametrize("steps", [1, 7, 8, 9, 11, 1025])
+def test_gdn_core_steps_lengths(ctx, steps):
+    """Core steps around the one-launch recurrence / token kernels line (8),
+    partial four-token chunks and more than one pass (1024): outputs, state and
+    windows are the bits of as many single core steps."""
+    rng = np.random.default_rng(steps)
+    heads, head, kernel = 16, 128, 4
+    layer, ws, conv_w, ssm_a, ssm_dt, conv = gdn_layer_for_core(ctx, rng)
+    state = (rng.standard_normal(heads * head * head) * 0.02).astype(np.float32)
+    cstate = (rng.standard_normal((kernel - 1) * conv) * 0.5).astype(np.float32)
+    rows = [rng.standard_normal((steps, n)).astype(np.float32) for n in (conv, heads, heads)]
+    bufs = [ctx.upload_array(a) for a in rows] + [ctx.alloc(steps * heads * head * 4) for _ in range(2)]
+    q, a, b, one, many = bufs
+    at = lambda buf, t, n: buf.ptr.value + t * n * 4
+    bits = lambda x: np.asarray(x, np.float32).view(np.uint32)
+    layer.set_state(state, cstate)
+    for t in range(steps):
+        ctx.call("fortai_hip_qwen35_recurrent_core_device", layer.h, at(q, t, conv), at(a, t, heads), at(b, t, heads),
+                 at(one, t, heads * head))
+    want, want_state = one.download(np.float32), layer.state()
+    layer.set_state(state, cstate)
+    ctx.call("fortai_hip_qwen35_recurrent_core_steps_device", layer.h, q.ptr, a.ptr, b.ptr, steps, many.ptr)
+    got, got_state = many.download(np.float32), layer.state()
+    assert np.array_equal(bits(got), bits(want))
+    assert all(np.array_equal(bits(x), bits(y)) for x, y in zip(got_state, want_state))
+    for buf in bufs:
+        buf.free()
+    layer.free()
+    for w in ws:
+        w.free()
