@@ -452,6 +452,15 @@ __device__ __forceinline__ uint32_t quantize_group(float4 y, float &scale_out, u
     return q0 | (q1 << 8) | (q2 << 16) | (q3 << 24);
 }
 
+// One quantized group into the token-block layout X8 (mmq.hip): value group l
+// of block b of token t.
+__device__ __forceinline__ void x8_store(int8_t *xq, float *xs, int ld, int t, int b, int l, uint32_t packed,
+    float scale) {
+    const size_t ct = static_cast<size_t>(b >> 2) * ld + t;
+    reinterpret_cast<uint32_t *>(xq)[ct * 32 + l * 4 + (b & 3)] = packed;
+    if (l == 0) xs[ct * 4 + (b & 3)] = scale;
+}
+
 // One 16-byte Q8L chunk (4 blocks) of a row lane: the reference's per-block
 // acc = fma(f32(w_scale) * a_scale, (float)dot4(w, a), acc), block by block.
 // sum of the four int8 products of a and b.  Kept on the builtin: the

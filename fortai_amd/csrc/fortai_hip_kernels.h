@@ -174,8 +174,8 @@ hipError_t launch_step_embedding(const uint16_t *table16, const Q8Matrix *table8
 hipError_t launch_count_nonfinite_halves(const uint16_t *w, size_t n, unsigned int *count, hipStream_t stream);
 
 // ---- token blocks on the i8 matrix cores (mmq.hip) --------------------------
-// X8 token activations: [blocks_pad][ld][32] int8 then [blocks_pad][ld] f32
-// scales, ld = q8_tokens_ld(tokens), blocks_pad = 4 * ceil(width / 128).
+// X8 token activations: [blocks_pad / 4][ld][8 lane parts][4 blocks][4] int8
+// then [blocks_pad / 4][ld][4] f32 scales, ld = q8_tokens_ld(tokens), blocks_pad = 4 * ceil(width / 128).
 int q8_tokens_ld(int tokens);
 size_t q8_tokens_bytes(int tokens, int width);
 hipError_t launch_q8_quantize_tokens(const float *x, int tokens, int width, int ld_x, void *x8, hipStream_t stream);

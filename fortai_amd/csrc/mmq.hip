@@ -14,11 +14,15 @@
 // per-block int32 dots are bit-exact and exported for testing.
 //
 // Token activations ("X8", written by q8_quantize_tokens_kernel):
-//   q[(b * ld + t) * 32 + k]   int8 value k of block b of token t
-//   s[b * ld + t]              f32 scale (the fp16-rounded reference scale)
+//   q[(c * ld + t) * 128 + l * 16 + j * 4 + k]  int8 value 4 l + k of block 4 c + j of token t
+//   s[(c * ld + t) * 4 + j]                     its f32 scale (the fp16-rounded reference scale)
 // with ld = tokens rounded up to 128 and blocks padded to a multiple of 4;
 // padding holds zeros.  The int8 part precedes the scales in one buffer of
-// q8_tokens_bytes() bytes.
+// q8_tokens_bytes() bytes.  A chunk (four blocks) of a token is 128 contiguous
+// bytes, lane part by lane part as the decode layouts have it: one 16-byte
+// load gives a lane its part of four blocks, and the lines that a token tile's
+// readers share at the same moment lie on different L2 channels (block by
+// block they were 32 ld bytes apart, for 128 tokens always the same two).
 //
 // Weights stay in the decode layout (q8_kernels.hip): lanes 4h..4h+3 of a
 // row's 16-byte pieces hold its bytes 16h..16h+15 of four consecutive blocks,
@@ -27,6 +31,9 @@
 // so the products pair up whatever k order the instruction uses internally.
 #include "fortai_hip_internal.h"
 #include "fortai_hip_kernels.h"
+
+#include <algorithm>
+#include <type_traits>
 
 
 namespace fortai_hip {
@@ -84,10 +91,8 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
     const int twl = (wave & 1) * 64;   // wave's first token within the tile
     const int rwl = (wave >> 1) * 64;  // wave's first row within the tile
     const int chunks = w.chunks;
-    const size_t bstride = static_cast<size_t>(ld) * 32;  // bytes per block of X8
-
     // global sources of this thread's share of a chunk:
-    //  tokens: 4 blocks x 128 tokens x 2 halves = 1024 pieces, 4 per thread
+    //  tokens: 128 tokens x 8 lane parts = 1024 pieces, 4 per thread
     //  rows:   16 row groups x 64 lanes          = 1024 pieces, 4 per thread
     //  token scales: 512 floats, 2 per thread;  row scales: 128 x uint2, threads < 128
     const int g_last = w.row_groups - 1;
@@ -98,17 +103,15 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int p = tid + k * kMmqThreads;          // 0..1023
-            const int j = p >> 8, t = (p >> 1) & 127, hh = p & 1;
-            ra[k] = *reinterpret_cast<const u32x4_t *>(xq + static_cast<size_t>(4 * c + j) * bstride +
-                static_cast<size_t>(t0 + t) * 32 + hh * 16);
+            ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(c) * ld + t0) * 128 + p * 16);
             const int g = min((r0 >> 3) + (p >> 6), g_last);  // clamped; rows past the end are not stored
             // cached loads: every token tile of the launch re-reads these rows
             rb[k] = reinterpret_cast<const u32x4_t *>(w.quants)[(static_cast<size_t>(g) * chunks + c) * 64 + (p & 63)];
         }
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            const int p = tid + k * kMmqThreads;  // 0..511
-            rs[k] = xs[static_cast<size_t>(4 * c + (p >> 7)) * ld + t0 + (p & 127)];
+            const int p = tid + k * kMmqThreads;  // 0..511: token p / 4, block p % 4
+            rs[k] = xs[(static_cast<size_t>(c) * ld + t0) * 4 + p];
         }
         if (tid < kRowTile) {
             const int g = min((r0 >> 3) + (tid >> 3), g_last);
@@ -116,29 +119,23 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
         }
     };
     auto stash = [&](MmqStage &st) {
+        // piece p: token or row p / 8, bytes 4l..4l+3 (l = p % 8) of the four blocks
+        uint32_t *da = reinterpret_cast<uint32_t *>(&st.a[0][0][0]), *db = reinterpret_cast<uint32_t *>(&st.b[0][0][0]);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int p = tid + k * kMmqThreads;
-            const int j = p >> 8, t = (p >> 1) & 127, hh = p & 1;
-            *reinterpret_cast<u32x4_t *>(&st.a[j][t][half_slot(t, hh)]) = ra[k];
-        }
-        // row piece: row (p >> 6) * 8 + r, bytes 4l..4l+3 of the four blocks
-        uint32_t *dst = reinterpret_cast<uint32_t *>(&st.b[0][0][0]);
+            const int n = p >> 3, l = p & 7;
+            const int base = (n * 2 + half_slot(n, l >> 2)) * 4 + (l & 3);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int p = tid + k * kMmqThreads;
-            const int q = p & 63, r = q >> 3, l = q & 7;
-            const int row = (p >> 6) * 8 + r;
-            const int base = (row * 2 + half_slot(row, l >> 2)) * 4 + (l & 3);
-            dst[base] = rb[k].x;
-            dst[base + kRowTile * 8] = rb[k].y;
-            dst[base + 2 * kRowTile * 8] = rb[k].z;
-            dst[base + 3 * kRowTile * 8] = rb[k].w;
+            for (int j = 0; j < 4; ++j) {
+                da[base + j * kTokTile * 8] = ra[k][j];
+                db[base + j * kRowTile * 8] = rb[k][j];
+            }
         }
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const int p = tid + k * kMmqThreads;
-            st.as[p >> 7][p & 127] = rs[k];
+            st.as[p & 3][p >> 2] = rs[k];
         }
         if (tid < kRowTile) {
             st.bs[0][tid] = half_bits_to_float(static_cast<uint16_t>(rws.x & 0xffffu));
@@ -301,11 +298,10 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
     const int twl = (wave & 1) * 32;   // wave's first token within the tile
     const int rwl = (wave >> 1) * 32;  // wave's first row within the tile
     const int chunks = w.chunks;
-    const size_t bstride = static_cast<size_t>(ld) * 32;  // bytes per block of X8
     const int g_last = w.row_groups - 1;
 
     // this thread's share of a chunk:
-    //   tokens: 4 blocks x 64 tokens x 2 halves = 512 pieces of 16 bytes, 2 per thread
+    //   tokens: 64 tokens x 8 lane parts        = 512 pieces of 16 bytes, 2 per thread
     //   rows:   8 row groups x 64 lanes         = 512 pieces of 16 bytes, 2 per thread
     //   token scales: 256 floats, 1 per thread; row scales: 64 x uint2, threads < 64
     u32x4_t ra[2], rb[2];
@@ -315,15 +311,11 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const int p = tid + k * kXThreads;  // 0..511
-            // a wave takes one (block, half) and 64 tokens, lane = token, so
-            // that its LDS stores (rows 18 dwords apart) meet no bank twice
-            const int j = p >> 7, hh = (p >> 6) & 1, t = p & 63;
-            ra[k] = *reinterpret_cast<const u32x4_t *>(xq + static_cast<size_t>(4 * c + j) * bstride +
-                static_cast<size_t>(t0 + t) * 32 + hh * 16);
+            ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(c) * ld + t0) * 128 + p * 16);
             const int g = min((r0 >> 3) + (p >> 6), g_last);  // clamped; rows past the end are not stored
             rb[k] = reinterpret_cast<const u32x4_t *>(w.quants)[(static_cast<size_t>(g) * chunks + c) * 64 + (p & 63)];
         }
-        rs = xs[static_cast<size_t>(4 * c + (tid >> 6)) * ld + t0 + (tid & 63)];
+        rs = xs[(static_cast<size_t>(c) * ld + t0) * 4 + tid];  // token tid / 4, block tid % 4
         if (tid < kXTile) {
             const int g = min((r0 >> 3) + (tid >> 3), g_last);
             rws = w.scales[(static_cast<size_t>(g) * chunks + c) * 8 + (tid & 7)];
@@ -332,24 +324,16 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
     auto stash = [&](MmqExactStage &st) {
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
+            // piece p: token or row p / 8, lane part p % 8 of the four blocks
             const int p = tid + k * kXThreads;
-            const int j = p >> 7, hh = (p >> 6) & 1, t = p & 63;
-            const uint32_t wd[4] = {ra[k].x, ra[k].y, ra[k].z, ra[k].w};
+            const int n = p >> 3, l = p & 7;
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
-                *reinterpret_cast<h4 *>(&st.a[j][t][part_slot(4 * hh + m)]) = i8x4_to_h4(wd[m]);
+            for (int j = 0; j < 4; ++j) {
+                *reinterpret_cast<h4 *>(&st.a[j][n][part_slot(l)]) = i8x4_to_h4(ra[k][j]);
+                *reinterpret_cast<h4 *>(&st.b[j][n][part_slot(l)]) = i8x4_to_h4(rb[k][j]);
+            }
         }
-#pragma unroll
-        for (int k = 0; k < 2; ++k) {
-            // row piece: row (p >> 6) * 8 + r, lane part l of the four blocks
-            const int p = tid + k * kXThreads;
-            const int q = p & 63, r = q >> 3, l = q & 7;
-            const int row = (p >> 6) * 8 + r;
-            const uint32_t wd[4] = {rb[k].x, rb[k].y, rb[k].z, rb[k].w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) *reinterpret_cast<h4 *>(&st.b[j][row][part_slot(l)]) = i8x4_to_h4(wd[j]);
-        }
-        st.as[tid >> 6][tid & 63] = rs;
+        st.as[tid & 3][tid >> 2] = rs;
         if (tid < kXTile) {
             st.bs[0][tid] = half_bits_to_float(static_cast<uint16_t>(rws.x & 0xffffu));
             st.bs[1][tid] = half_bits_to_float(static_cast<uint16_t>(rws.x >> 16));
@@ -437,6 +421,138 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
     }
 }
 
+// The same product for few tokens or few rows, where 64 x 64 tiles leave most
+// CUs idle and a wave's 32 x 32 x 8 chains make each chunk a long serial
+// stretch: a wave takes 16 rows, TT x 16 tokens and four of the eight lane
+// parts (g = wave & 1: parts 4 g .. 4 g + 3), so a quadrant's chains are spread
+// over two waves and a block costs a wave TT matrix instructions.  No LDS
+// before the end: the decode layout already holds, for lane (row, part), the
+// bytes of four blocks in 16 contiguous bytes, the B operand of four
+// instructions, and a token's part is one dword of X8; both are widened in
+// registers.  The waves of a workgroup meet once, when wave g = 1 hands its
+// chains to wave g = 0 for the horizontal sum.  Operands are loaded
+// kSmallAhead chunks ahead (the weights come from HBM).  With the quantizer's
+// launch, same bits, 64 x 64 tiles before: 2560 x 9216, 16 tokens 151 -> 29 us;
+// 1024 x 3584, 77 tokens 63 -> 15 us; 32 x 2560, 4096 tokens 57 -> 22 us;
+// 9216 x 2560, 33 tokens 46 -> 29 us.
+constexpr int kSmallRows = 32;   // rows per workgroup: two wave pairs of 16
+
+constexpr int kSmallAhead = 4;   // chunks in flight (8: the same, with more registers)
+
+template <int TT, int EPI>
+__global__ __launch_bounds__(256, 2) void q8_mmq_exact_small_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
+    const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
+    const float *__restrict__ resid, int token_tiles) {
+    __shared__ float hand[2][TT * 16][64];
+    __shared__ __align__(16) float scales[4][TT][64];  // per wave: a chunk's token scales [block][token]
+    const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
+    const int g = wave & 1, pair = wave >> 1;
+    const int i = lane & 15, s4 = lane >> 4;
+    // workgroup b runs on XCD b % 8: with eight row tiles or more, the token
+    // tiles of a row tile are consecutive there, so its L2 serves them the
+    // weights; fewer row tiles would leave XCDs idle that way
+    const int id = static_cast<int>(blockIdx.x);
+    const bool grouped = w.rows > 7 * kSmallRows;  // (w.rows + 31) / 32 >= 8, as the launch has it
+    const int row_tile = grouped ? id / 8 / token_tiles * 8 + id % 8 : id / token_tiles;
+    const int t0 = (grouped ? id / 8 % token_tiles : id % token_tiles) * (16 * TT);
+    if (row_tile * kSmallRows >= w.rows) return;  // (the grid is padded to whole groups of eight)
+    const int row = row_tile * kSmallRows + 16 * pair + i;
+    const int chunks = w.chunks;
+    const int g8 = min(row >> 3, w.row_groups - 1);  // clamped; rows past the end are not stored
+    const u32x4_t *wq = reinterpret_cast<const u32x4_t *>(w.quants) + static_cast<size_t>(g8) * chunks * 64 + (row & 7) * 8 + s4 + 4 * g;
+    const uint2 *ws = w.scales + static_cast<size_t>(g8) * chunks * 8 + (row & 7);
+    // this lane's token and part; token lane / 4, block lane % 4 of the scales
+    const u32x4_t *aq = reinterpret_cast<const u32x4_t *>(xq) + static_cast<size_t>(t0 + i) * 8 + s4 + 4 * g;
+    const float *as = xs + static_cast<size_t>(t0) * 4 + lane;
+
+    u32x4_t bq[kSmallAhead];
+    uint2 bs[kSmallAhead];
+    u32x4_t av[kSmallAhead][TT];
+    float at[kSmallAhead][TT];
+    auto fetch = [&](int c, int slot) {
+        const int cc = min(c, chunks - 1);
+        const size_t b = static_cast<size_t>(cc) * ld;
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) {
+            at[slot][tt] = as[b * 4 + tt * 64];
+            av[slot][tt] = aq[b * 8 + tt * 128];
+        }
+        bq[slot] = wq[static_cast<size_t>(cc) * 64];
+        bs[slot] = ws[static_cast<size_t>(cc) * 8];
+    };
+    float acc[TT][16];
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[tt][r] = 0.0f;
+    auto consume = [&](const u32x4_t &q4, const uint2 &sc, const u32x4_t (&a)[TT], const float (&asc)[TT]) {
+        // the wave's own LDS, in order: no barrier
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt) scales[wave][tt][16 * (lane & 3) + (lane >> 2)] = asc[tt];
+        wave_lds_fence();
+        const f32x16 zero = {};
+        f32x16 d = __builtin_amdgcn_mfma_f32_16x16x4f16(i8x4_to_h4(a[0][0]), i8x4_to_h4(q4[0]), zero, 0, 0, 0);
+#pragma unroll
+        for (int m = 0; m < 4 * TT; ++m) {  // block m / TT, token tile m % TT; each product issued before the last one's fmas
+            const int j = m / TT, tt = m % TT;
+            f32x16 dn = zero;
+            if (m + 1 < 4 * TT) {
+                const int j1 = (m + 1) / TT, tt1 = (m + 1) % TT;
+                dn = __builtin_amdgcn_mfma_f32_16x16x4f16(i8x4_to_h4(a[tt1][j1]), i8x4_to_h4(q4[j1]), zero, 0, 0, 0);
+            }
+            const uint32_t sh = j < 2 ? sc.x : sc.y;
+            const float4 x = *reinterpret_cast<const float4 *>(&scales[wave][tt][16 * j + 4 * s4]);
+            // fl(f32(w_scale) * x_scale) of this lane's four tokens
+            const float p[4] = {j & 1 ? half_times<true>(sh, x.x) : half_times<false>(sh, x.x),
+                j & 1 ? half_times<true>(sh, x.y) : half_times<false>(sh, x.y),
+                j & 1 ? half_times<true>(sh, x.z) : half_times<false>(sh, x.z),
+                j & 1 ? half_times<true>(sh, x.w) : half_times<false>(sh, x.w)};
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[tt][r] = __builtin_fmaf(p[r & 3], d[r], acc[tt][r]);
+            d = dn;
+        }
+        wave_lds_fence();
+    };
+#pragma unroll
+    for (int k = 0; k < kSmallAhead; ++k) fetch(k, k);
+    int c = 0;
+    for (; c + kSmallAhead <= chunks; c += kSmallAhead) {
+#pragma unroll
+        for (int k = 0; k < kSmallAhead; ++k) {
+            __builtin_amdgcn_sched_barrier(0);
+            consume(bq[k], bs[k], av[k], at[k]);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(c + k + kSmallAhead, k);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kSmallAhead - 1; ++k)
+        if (c + k < chunks) consume(bq[k], bs[k], av[k], at[k]);  // uniform
+    if (g == 1) {
+#pragma unroll
+        for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) hand[pair][tt * 16 + r][lane] = acc[tt][r];
+    }
+    __syncthreads();
+    if (g == 1 || row >= w.rows) return;
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int t = t0 + 16 * tt + 4 * s4 + u;
+            if (t >= tokens) continue;
+            // chain L of token u: register 4 (L % 4) + u of wave g = L / 4; the
+            // horizontal sum of fortai_q8_dot.c:323-330
+            auto lo = [&](int L) { return acc[tt][4 * L + u]; };
+            auto hi = [&](int L) { return hand[pair][tt * 16 + 4 * L + u][lane]; };
+            const float sum = ((lo(0) + hi(0)) + (lo(2) + hi(2))) + ((lo(1) + hi(1)) + (lo(3) + hi(3)));
+            const size_t o = static_cast<size_t>(t) * ld_out + row;
+            if constexpr (EPI == 1) out[o] = sum + resid[o];
+            else out[o] = sum;
+        }
+}
+
 // fortai_q8_quantize (fortai_q8_dot.c:153-198) of every token into X8: one
 // thread per 4 values, 8 consecutive threads per block.
 __global__ __launch_bounds__(256) void q8_quantize_tokens_kernel(const float *__restrict__ x, int tokens, int width,
@@ -451,8 +567,7 @@ __global__ __launch_bounds__(256) void q8_quantize_tokens_kernel(const float *__
     uint16_t bits;
     const uint32_t packed = quantize_group(y, scale, bits);
     const int b = g >> 3, l = g & 7;
-    reinterpret_cast<uint32_t *>(xq + (static_cast<size_t>(b) * ld + t) * 32)[l] = packed;
-    if (l == 0) xs[static_cast<size_t>(b) * ld + t] = scale;
+    x8_store(xq, xs, ld, t, b, l, packed, scale);
 }
 
 }  // namespace
@@ -483,6 +598,36 @@ hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, fl
     const int8_t *xq = static_cast<const int8_t *>(x8);
     const float *xs = reinterpret_cast<const float *>(xq + static_cast<size_t>(ld) * w.chunks * 4 * 32);
     const dim3 grid((w.rows + kXTile - 1) / kXTile, (tokens + kXTile - 1) / kXTile);
+    // Time per chunk (four blocks of width) by workgroups per CU, us, measured
+    // over rows 16 .. 9216, widths 1024 .. 9216 and 1 .. 1200 tokens: 64 x 64
+    // tiles 2.15 while each CU has at most one, then 3.1 for two and 1.6 for
+    // each more; 32 rows x 16 tokens 0.15 + 0.29 each, x 32 tokens 0.25 + 0.47
+    // each (a workgroup of either does 1/8 or 1/4 of the large one's work).
+    constexpr int kCus = 256;
+    auto per_cu = [&](int row_tile, int token_tile) {
+        const long long wgs = static_cast<long long>((w.rows + row_tile - 1) / row_tile) * ((tokens + token_tile - 1) / token_tile);
+        return static_cast<double>((wgs + kCus - 1) / kCus);
+    };
+    const double nb = per_cu(kXTile, kXTile);
+    const double large = nb <= 1.0 ? 2.15 : std::max(3.1, 1.6 * nb);
+    const double one = 0.15 + 0.29 * per_cu(kSmallRows, 16), two = 0.25 + 0.47 * per_cu(kSmallRows, 32);
+    if (std::min(one, two) < large) {
+        auto small = [&](auto tt_c) {
+            constexpr int TT = decltype(tt_c)::value;
+            const int tt_n = (tokens + 16 * TT - 1) / (16 * TT), rt_n = (w.rows + kSmallRows - 1) / kSmallRows;
+            const dim3 sgrid((rt_n >= 8 ? (rt_n + 7) / 8 * 8 : rt_n) * tt_n);
+            if (resid)
+                hipLaunchKernelGGL((q8_mmq_exact_small_kernel<TT, 1>), sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld,
+                    out, ld_out, resid, tt_n);
+            else
+                hipLaunchKernelGGL((q8_mmq_exact_small_kernel<TT, 0>), sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld,
+                    out, ld_out, resid, tt_n);
+            note_launch("q8_mmq_exact_small_kernel<%d,%s> grid %d", TT, resid ? "add" : "store", sgrid.x);
+        };
+        if (one <= two) small(std::integral_constant<int, 1>{});
+        else small(std::integral_constant<int, 2>{});
+        return hipGetLastError();
+    }
     const size_t lds = 2 * sizeof(MmqExactStage);
     if (resid)
         hipLaunchKernelGGL((q8_mmq_exact_kernel<1>), grid, dim3(kXThreads), lds, stream, w, xq, xs, tokens, ld, out,

@@ -56,8 +56,7 @@ __global__ __launch_bounds__(kRowThreads) void rms_quantize_tokens_kernel(const 
         uint16_t bits;
         const uint32_t packed = quantize_group(y, scale, bits);
         const int b = g >> 3, l = g & 7;
-        reinterpret_cast<uint32_t *>(xq + (static_cast<size_t>(b) * ld + n) * 32)[l] = packed;
-        if (l == 0) xs[static_cast<size_t>(b) * ld + n] = scale;
+        x8_store(xq, xs, ld, n, b, l, packed, scale);
     }
 }
 
@@ -92,8 +91,7 @@ __global__ __launch_bounds__(kRowThreads) void gated_quantize_tokens_kernel(cons
         const uint32_t packed = quantize_group(y, scale, bits);
         if (g < blocks_pad * 8) {
             const int b = g >> 3, l = g & 7;
-            reinterpret_cast<uint32_t *>(xq + (static_cast<size_t>(b) * ld + n) * 32)[l] = packed;
-            if (l == 0) xs[static_cast<size_t>(b) * ld + n] = scale;
+            x8_store(xq, xs, ld, n, b, l, packed, scale);
         }
     }
 }
@@ -114,8 +112,7 @@ __global__ __launch_bounds__(kRowThreads) void silu_product_quantize_kernel(cons
         uint16_t bits;
         const uint32_t packed = quantize_group(y, scale, bits);
         const int b = g >> 3, l = g & 7;
-        reinterpret_cast<uint32_t *>(xq + (static_cast<size_t>(b) * ld + n) * 32)[l] = packed;
-        if (l == 0) xs[static_cast<size_t>(b) * ld + n] = scale;
+        x8_store(xq, xs, ld, n, b, l, packed, scale);
     }
 }
 
@@ -1115,11 +1112,10 @@ __global__ __launch_bounds__(256) void x8_to_q8l_kernel(const int8_t *__restrict
     uint32_t *dst = q8l + static_cast<size_t>(rr) * chunks * 36;
     for (int e = static_cast<int>(threadIdx.x); e < chunks * 36; e += 256) {
         if (e < chunks * 32) {
-            const int c = e >> 5, l = (e >> 2) & 7, j = e & 3, b = 4 * c + j;
-            dst[e] = reinterpret_cast<const uint32_t *>(xq + (static_cast<size_t>(b) * ld + n) * 32)[l];
+            dst[e] = reinterpret_cast<const uint32_t *>(xq + (static_cast<size_t>(e >> 5) * ld + n) * 128)[e & 31];
         } else {
             const int b = e - chunks * 32;
-            reinterpret_cast<float *>(dst)[e] = xs[static_cast<size_t>(b) * ld + n];
+            reinterpret_cast<float *>(dst)[e] = xs[(static_cast<size_t>(b >> 2) * ld + n) * 4 + (b & 3)];
         }
     }
 }

@@ -132,3 +132,35 @@ def test_mmq_lane_order_bit_identical(ctx, oracle, rows, width, tokens):
     ctx.call("fortai_hip_q8_mmq_exact_device", ctx.h, W.h, dq.ptr, tokens, dr.ptr, dr.ptr, None)
     assert np.array_equal(dr.download(np.float32).reshape(tokens, rows), (got + resid).astype(np.float32))
     W.free()
+
+
+@pytest.mark.parametrize("rows,width,tokens", [(1, 32, 1), (32, 128, 16), (33, 640, 17), (224, 512, 33), (225, 544, 31),
+                                               (264, 1664, 48), (300, 96, 260), (17, 2560, 300), (2560, 1056, 150),
+                                               (4100, 160, 200), (2100, 96, 900)])
+def test_mmq_lane_order_tiles(ctx, rows, width, tokens):
+    """The token product's tile choices -- 64 x 64, 32 rows x 16 and x 32
+    tokens, fewer and more than eight row tiles, ragged rows and tokens, whole
+    and partial groups of four chunks -- against the batched matvec of the same
+    tokens (itself checked against the oracle), bit for bit, with and without
+    the residual."""
+    rng = np.random.default_rng(rows + 3 * width + tokens)
+    W = B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    x = rng.standard_normal((tokens, width)).astype(np.float32)
+    x[tokens // 2, :32] = 0.0
+    dx = ctx.upload_array(x)
+    dq = ctx.alloc(B.load().fortai_hip_q8_tokens_bytes(tokens, width))
+    out, want = ctx.alloc(tokens * rows * 4), ctx.alloc(tokens * rows * 4)
+    for t in range(0, tokens, 8):
+        ctx.call("fortai_hip_q8_batch_matvec_device", ctx.h, W.h, dx.ptr.value + t * width * 4, min(8, tokens - t),
+                 want.ptr.value + t * rows * 4, None)
+    ctx.call("fortai_hip_q8_quantize_tokens_device", ctx.h, dx.ptr, tokens, width, dq.ptr)
+    ctx.call("fortai_hip_q8_mmq_exact_device", ctx.h, W.h, dq.ptr, tokens, out.ptr, None, None)
+    expect = want.download(np.float32)
+    assert np.array_equal(out.download(np.float32).view(np.uint32), expect.view(np.uint32))
+    resid = rng.standard_normal(tokens * rows).astype(np.float32)
+    out.upload(resid)
+    ctx.call("fortai_hip_q8_mmq_exact_device", ctx.h, W.h, dq.ptr, tokens, out.ptr, out.ptr, None)
+    assert np.array_equal(out.download(np.float32).view(np.uint32), (expect + resid).view(np.uint32))
+    for b in (dx, dq, out, want):
+        b.free()
+    W.free()
