@@ -1004,7 +1004,7 @@ int fortai_hip_q8_mmq_device(fortai_hip_q8_context *c, const fortai_hip_q8_weigh
     if (kernel_ms) e = hipEventRecord(c->start, c->stream);
     if (e == hipSuccess)
         e = launch_q8_mmq(w->m, x8, tokens, static_cast<float *>(out), w->m.rows, static_cast<const float *>(resid),
-            nullptr, c->stream);
+            nullptr, X8Layout::BLOCKS, c->stream);
     if (kernel_ms) {
         if (e == hipSuccess) e = hipEventRecord(c->stop, c->stream);
         if (e == hipSuccess) e = hipEventSynchronize(c->stop);
@@ -1021,7 +1021,7 @@ int fortai_hip_q8_mmq_exact_device(fortai_hip_q8_context *c, const fortai_hip_q8
     if (kernel_ms) e = hipEventRecord(c->start, c->stream);
     if (e == hipSuccess)
         e = launch_q8_mmq_exact(w->m, x8, tokens, static_cast<float *>(out), w->m.rows,
-            static_cast<const float *>(resid), c->stream);
+            static_cast<const float *>(resid), X8Layout::BLOCKS, c->stream);
     if (kernel_ms) {
         if (e == hipSuccess) e = hipEventRecord(c->stop, c->stream);
         if (e == hipSuccess) e = hipEventSynchronize(c->stop);
@@ -1037,7 +1037,7 @@ int fortai_hip_q8_mmq_block_dots(fortai_hip_q8_context *c, const fortai_hip_q8_w
     float *scratch = nullptr;
     hipError_t e = hipMalloc(&scratch, static_cast<size_t>(tokens) * w->m.rows * sizeof(float));
     if (e == hipSuccess)
-        e = launch_q8_mmq(w->m, x8, tokens, scratch, w->m.rows, nullptr, static_cast<int32_t *>(dots), c->stream);
+        e = launch_q8_mmq(w->m, x8, tokens, scratch, w->m.rows, nullptr, static_cast<int32_t *>(dots), X8Layout::BLOCKS, c->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (scratch) (void)hipFree(scratch);
     return done(c, e, "token-block dots");
@@ -2333,8 +2333,9 @@ hipError_t enqueue_batch_prefill(fortai_hip_qwen35_batch *b, int T, PrefillMode 
                                 : launch_q8_embedding(b->emb8->m, b->ptokens, 0, b->px, stream, N), "token embeddings");
     auto mmq = [&](const fortai_hip_q8_weights *w, float *out, const float *resid, const char *op) {
         if (mode == PrefillMode::EXACT)
-            return rec(launch_q8_mmq_exact(w->m, b->px8, N, out, w->m.rows, resid, stream), op);
-        if (mode == PrefillMode::FAST) return rec(launch_q8_mmq(w->m, b->px8, N, out, w->m.rows, resid, nullptr, stream), op);
+            return rec(launch_q8_mmq_exact(w->m, b->px8, N, out, w->m.rows, resid, X8Layout::CHUNKS, stream), op);
+        if (mode == PrefillMode::FAST) 
+            return rec(launch_q8_mmq(w->m, b->px8, N, out, w->m.rows, resid, nullptr, X8Layout::CHUNKS, stream), op);
         hipError_t r = hipSuccess;
         for (int r0 = 0; r0 < N && r == hipSuccess; r0 += 8) {
             const int cnt = std::min(8, N - r0);

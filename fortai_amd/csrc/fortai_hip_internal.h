@@ -452,7 +452,7 @@ __device__ __forceinline__ uint32_t quantize_group(float4 y, float &scale_out, u
     return q0 | (q1 << 8) | (q2 << 16) | (q3 << 24);
 }
 
-// One quantized group into the token-block layout X8 (mmq.hip): value group l
+// One quantized group into the chunk-major token layout X8 (mmq.hip): value group l
 // of block b of token t.
 __device__ __forceinline__ void x8_store(int8_t *xq, float *xs, int ld, int t, int b, int l, uint32_t packed,
     float scale) {

@@ -174,19 +174,23 @@ hipError_t launch_step_embedding(const uint16_t *table16, const Q8Matrix *table8
 hipError_t launch_count_nonfinite_halves(const uint16_t *w, size_t n, unsigned int *count, hipStream_t stream);
 
 // ---- token blocks on the i8 matrix cores (mmq.hip) --------------------------
-// X8 token activations: [blocks_pad / 4][ld][8 lane parts][4 blocks][4] int8
-// then [blocks_pad / 4][ld][4] f32 scales, ld = q8_tokens_ld(tokens), blocks_pad = 4 * ceil(width / 128).
+// X8 token activations, ld = q8_tokens_ld(tokens), blocks_pad = 4 * ceil(width / 128):
+//  BLOCKS (the entry points): [blocks_pad][ld][32] int8, then [blocks_pad][ld] f32 scales;
+//  CHUNKS (inside the prefill): [blocks_pad / 4][ld][8 lane parts][4 blocks][4] int8,
+//  then [blocks_pad / 4][ld][4] f32 scales.
+enum class X8Layout { BLOCKS, CHUNKS };
 int q8_tokens_ld(int tokens);
 size_t q8_tokens_bytes(int tokens, int width);
+// (block-major)
 hipError_t launch_q8_quantize_tokens(const float *x, int tokens, int width, int ld_x, void *x8, hipStream_t stream);
 // out[t * ld_out + row] = W . x_t (+ resid at the same index); optional
-// int32 block dots [tokens][rows][blocks]
+// int32 block dots [tokens][rows][blocks] (block-major X8 only)
 hipError_t launch_q8_mmq(const Q8Matrix &w, const void *x8, int tokens, float *out, int ld_out, const float *resid,
-    int32_t *dots, hipStream_t stream);
+    int32_t *dots, X8Layout layout, hipStream_t stream);
 // The same product with the reference's eight-lane fp32 order kept: every
 // output is bit-identical to the decode matvec of its token.
 hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, float *out, int ld_out,
-    const float *resid, hipStream_t stream);
+    const float *resid, X8Layout layout, hipStream_t stream);
 
 // ---- Gated DeltaNet ------------------------------------------------------
 struct GdnParams {
@@ -264,15 +268,15 @@ bool attention_quantizes_output(const AttentionParams &p, int batch);
 size_t attention_scores_floats(int heads, int max_context);
 
 // ---- prompt prefill (prefill.hip): rows are tokens, row s * T + t ---------------
-// rows [r0, r0 + count) of an X8 buffer -> Q8L [count][q8l_bytes(width)]
+// rows [r0, r0 + count) of a chunk-major X8 buffer -> Q8L [count][q8l_bytes(width)]
 hipError_t launch_x8_to_q8l(const void *x8, int tokens, int width, int r0, int count, void *q8l, hipStream_t stream);
-// x [rows][width] -> optional RMSNorm -> X8 (q8_tokens_bytes(rows, width))
+// x [rows][width] -> optional RMSNorm -> chunk-major X8 (q8_tokens_bytes(rows, width))
 hipError_t launch_rms_quantize_tokens(const float *x, int rows, int width, const float *norm, float eps, void *x8,
     hipStream_t stream);
-// GDN o and raw gate z [rows][width] -> per-head gated RMSNorm -> X8
+// GDN o and raw gate z [rows][width] -> per-head gated RMSNorm -> chunk-major X8
 hipError_t launch_gated_quantize_tokens(const float *o, const float *z, const float *norm, float eps, int rows,
     int width, int head, void *x8, hipStream_t stream);
-// silu(gate) * up [rows][width] -> X8
+// silu(gate) * up [rows][width] -> chunk-major X8
 hipError_t launch_silu_product_quantize(const float *gate, const float *up, int rows, int width, void *x8,
     hipStream_t stream);
 // causal conv1d + SiLU over T tokens of every sequence, continuing conv_state

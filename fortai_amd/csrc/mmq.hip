@@ -13,16 +13,21 @@
 // agree with it to fp32 rounding (relative 1e-5 class), not bit for bit; the
 // per-block int32 dots are bit-exact and exported for testing.
 //
-// Token activations ("X8", written by q8_quantize_tokens_kernel):
+// Token activations ("X8") come in two layouts of the same size.  Block-major,
+// written by q8_quantize_tokens_kernel and read by the entry points:
+//   q[(b * ld + t) * 32 + k]   int8 value k of block b of token t
+//   s[b * ld + t]              f32 scale (the fp16-rounded reference scale)
+// Chunk-major, written and read inside the prompt prefill:
 //   q[(c * ld + t) * 128 + l * 16 + j * 4 + k]  int8 value 4 l + k of block 4 c + j of token t
-//   s[(c * ld + t) * 4 + j]                     its f32 scale (the fp16-rounded reference scale)
+//   s[(c * ld + t) * 4 + j]                     its scale
 // with ld = tokens rounded up to 128 and blocks padded to a multiple of 4;
 // padding holds zeros.  The int8 part precedes the scales in one buffer of
-// q8_tokens_bytes() bytes.  A chunk (four blocks) of a token is 128 contiguous
-// bytes, lane part by lane part as the decode layouts have it: one 16-byte
-// load gives a lane its part of four blocks, and the lines that a token tile's
-// readers share at the same moment lie on different L2 channels (block by
-// block they were 32 ld bytes apart, for 128 tokens always the same two).
+// q8_tokens_bytes() bytes.  Chunk-major, a token's chunk (four blocks) is 128
+// contiguous bytes, lane part by lane part as the decode layouts have it: one
+// 16-byte load gives a lane its part of four blocks, and the lines that a token
+// tile's readers share at the same moment lie on different L2 channels
+// (block-major they are 32 ld bytes apart: for up to 128 tokens always the
+// same two).
 //
 // Weights stay in the decode layout (q8_kernels.hip): lanes 4h..4h+3 of a
 // row's 16-byte pieces hold its bytes 16h..16h+15 of four consecutive blocks,
@@ -75,9 +80,10 @@ __device__ __forceinline__ int half_slot(int n, int h) { return h ^ ((n >> 3) & 
 // rows 64 (w >> 1) as 2 x 2 MFMA tiles of 32 x 32.  Chunk c + 1 is loaded
 // into registers while chunk c is consumed from LDS, then stored to the other
 // stage (one barrier per chunk).
+//   BLOCKS: X8 block-major, else chunk-major
 //   EPI 0: out[t * ld_out + row] = acc;  EPI 1: out = acc + resid (same index)
 //   DOTS: also write every int32 block dot to dots[(t * rows + row) * blocks + b]
-template <int EPI, bool DOTS>
+template <int EPI, bool DOTS, bool BLOCKS>
 __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
     const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
     const float *__restrict__ resid, int32_t *__restrict__ dots) {
@@ -92,7 +98,7 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
     const int rwl = (wave >> 1) * 64;  // wave's first row within the tile
     const int chunks = w.chunks;
     // global sources of this thread's share of a chunk:
-    //  tokens: 128 tokens x 8 lane parts = 1024 pieces, 4 per thread
+    //  tokens: 128 tokens x 8 lane parts (BLOCKS: 4 blocks x 128 tokens x 2 halves) = 1024 pieces, 4 per thread
     //  rows:   16 row groups x 64 lanes          = 1024 pieces, 4 per thread
     //  token scales: 512 floats, 2 per thread;  row scales: 128 x uint2, threads < 128
     const int g_last = w.row_groups - 1;
@@ -103,15 +109,19 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int p = tid + k * kMmqThreads;          // 0..1023
-            ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(c) * ld + t0) * 128 + p * 16);
+            if constexpr (BLOCKS)  // block p / 256, token p / 2 % 128, half p % 2
+                ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(4 * c + (p >> 8)) * ld + t0) * 32 + (p & 255) * 16);
+            else
+                ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(c) * ld + t0) * 128 + p * 16);
             const int g = min((r0 >> 3) + (p >> 6), g_last);  // clamped; rows past the end are not stored
             // cached loads: every token tile of the launch re-reads these rows
             rb[k] = reinterpret_cast<const u32x4_t *>(w.quants)[(static_cast<size_t>(g) * chunks + c) * 64 + (p & 63)];
         }
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
-            const int p = tid + k * kMmqThreads;  // 0..511: token p / 4, block p % 4
-            rs[k] = xs[(static_cast<size_t>(c) * ld + t0) * 4 + p];
+            const int p = tid + k * kMmqThreads;  // 0..511: token p / 4, block p % 4 (BLOCKS: block p / 128, token p % 128)
+            rs[k] = BLOCKS ? xs[static_cast<size_t>(4 * c + (p >> 7)) * ld + t0 + (p & 127)]
+                           : xs[(static_cast<size_t>(c) * ld + t0) * 4 + p];
         }
         if (tid < kRowTile) {
             const int g = min((r0 >> 3) + (tid >> 3), g_last);
@@ -126,16 +136,19 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
             const int p = tid + k * kMmqThreads;
             const int n = p >> 3, l = p & 7;
             const int base = (n * 2 + half_slot(n, l >> 2)) * 4 + (l & 3);
+            if constexpr (BLOCKS)
+                *reinterpret_cast<u32x4_t *>(&st.a[p >> 8][(p >> 1) & 127][half_slot((p >> 1) & 127, p & 1)]) = ra[k];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                da[base + j * kTokTile * 8] = ra[k][j];
+                if constexpr (!BLOCKS) da[base + j * kTokTile * 8] = ra[k][j];
                 db[base + j * kRowTile * 8] = rb[k][j];
             }
         }
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const int p = tid + k * kMmqThreads;
-            st.as[p & 3][p >> 2] = rs[k];
+            if constexpr (BLOCKS) st.as[p >> 7][p & 127] = rs[k];
+            else st.as[p & 3][p >> 2] = rs[k];
         }
         if (tid < kRowTile) {
             st.bs[0][tid] = half_bits_to_float(static_cast<uint16_t>(rws.x & 0xffffu));
@@ -284,7 +297,7 @@ __device__ __forceinline__ h4 i8x4_to_h4(uint32_t w) {
     return h4{a.x, a.y, b.x, b.y};
 }
 
-template <int EPI>
+template <int EPI, bool BLOCKS>
 __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
     const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
     const float *__restrict__ resid) {
@@ -302,6 +315,8 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
 
     // this thread's share of a chunk:
     //   tokens: 64 tokens x 8 lane parts        = 512 pieces of 16 bytes, 2 per thread
+    //           (BLOCKS: a wave takes one block and half and 64 tokens, lane =
+    //           token, so that its LDS stores, rows 18 dwords apart, meet no bank twice)
     //   rows:   8 row groups x 64 lanes         = 512 pieces of 16 bytes, 2 per thread
     //   token scales: 256 floats, 1 per thread; row scales: 64 x uint2, threads < 64
     u32x4_t ra[2], rb[2];
@@ -311,11 +326,17 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
 #pragma unroll
         for (int k = 0; k < 2; ++k) {
             const int p = tid + k * kXThreads;  // 0..511
-            ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(c) * ld + t0) * 128 + p * 16);
+            if constexpr (BLOCKS)
+                ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(4 * c + (p >> 7)) * ld + t0 + (p & 63)) * 32 +
+                    ((p >> 6) & 1) * 16);
+            else
+                ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(c) * ld + t0) * 128 + p * 16);
             const int g = min((r0 >> 3) + (p >> 6), g_last);  // clamped; rows past the end are not stored
             rb[k] = reinterpret_cast<const u32x4_t *>(w.quants)[(static_cast<size_t>(g) * chunks + c) * 64 + (p & 63)];
         }
-        rs = xs[(static_cast<size_t>(c) * ld + t0) * 4 + tid];  // token tid / 4, block tid % 4
+        // token tid / 4, block tid % 4 (BLOCKS: block tid / 64, token tid % 64)
+        rs = BLOCKS ? xs[static_cast<size_t>(4 * c + (tid >> 6)) * ld + t0 + (tid & 63)]
+                    : xs[(static_cast<size_t>(c) * ld + t0) * 4 + tid];
         if (tid < kXTile) {
             const int g = min((r0 >> 3) + (tid >> 3), g_last);
             rws = w.scales[(static_cast<size_t>(g) * chunks + c) * 8 + (tid & 7)];
@@ -329,11 +350,15 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
             const int n = p >> 3, l = p & 7;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                *reinterpret_cast<h4 *>(&st.a[j][n][part_slot(l)]) = i8x4_to_h4(ra[k][j]);
+                if constexpr (BLOCKS)
+                    *reinterpret_cast<h4 *>(&st.a[p >> 7][p & 63][part_slot(4 * ((p >> 6) & 1) + j)]) = i8x4_to_h4(ra[k][j]);
+                else
+                    *reinterpret_cast<h4 *>(&st.a[j][n][part_slot(l)]) = i8x4_to_h4(ra[k][j]);
                 *reinterpret_cast<h4 *>(&st.b[j][n][part_slot(l)]) = i8x4_to_h4(rb[k][j]);
             }
         }
-        st.as[tid & 3][tid >> 2] = rs;
+        if constexpr (BLOCKS) st.as[tid >> 6][tid & 63] = rs;
+        else st.as[tid & 3][tid >> 2] = rs;
         if (tid < kXTile) {
             st.bs[0][tid] = half_bits_to_float(static_cast<uint16_t>(rws.x & 0xffffu));
             st.bs[1][tid] = half_bits_to_float(static_cast<uint16_t>(rws.x >> 16));
@@ -432,14 +457,15 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
 // registers.  The waves of a workgroup meet once, when wave g = 1 hands its
 // chains to wave g = 0 for the horizontal sum.  Operands are loaded
 // kSmallAhead chunks ahead (the weights come from HBM).  With the quantizer's
-// launch, same bits, 64 x 64 tiles before: 2560 x 9216, 16 tokens 151 -> 29 us;
-// 1024 x 3584, 77 tokens 63 -> 15 us; 32 x 2560, 4096 tokens 57 -> 22 us;
-// 9216 x 2560, 33 tokens 46 -> 29 us.
+// launch, same bits, 64 x 64 tiles before (chunk-major / block-major tokens):
+// 2560 x 9216, 16 tokens 151 -> 29 / 48 us; 1024 x 3584, 77 tokens 63 -> 15 /
+// 23 us; 32 x 2560, 4096 tokens 57 -> 22 / 23 us; 9216 x 2560, 33 tokens 46 -> 29 us
+// (block-major: the 64 x 64 tiles).
 constexpr int kSmallRows = 32;   // rows per workgroup: two wave pairs of 16
 
 constexpr int kSmallAhead = 4;   // chunks in flight (8: the same, with more registers)
 
-template <int TT, int EPI>
+template <int TT, int EPI, bool BLOCKS>
 __global__ __launch_bounds__(256, 2) void q8_mmq_exact_small_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
     const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
     const float *__restrict__ resid, int token_tiles) {
@@ -461,9 +487,11 @@ __global__ __launch_bounds__(256, 2) void q8_mmq_exact_small_kernel(Q8Matrix w, 
     const int g8 = min(row >> 3, w.row_groups - 1);  // clamped; rows past the end are not stored
     const u32x4_t *wq = reinterpret_cast<const u32x4_t *>(w.quants) + static_cast<size_t>(g8) * chunks * 64 + (row & 7) * 8 + s4 + 4 * g;
     const uint2 *ws = w.scales + static_cast<size_t>(g8) * chunks * 8 + (row & 7);
-    // this lane's token and part; token lane / 4, block lane % 4 of the scales
-    const u32x4_t *aq = reinterpret_cast<const u32x4_t *>(xq) + static_cast<size_t>(t0 + i) * 8 + s4 + 4 * g;
-    const float *as = xs + static_cast<size_t>(t0) * 4 + lane;
+    // this lane's token and part; of the scales, token lane / 4 and block
+    // lane % 4 (BLOCKS: block s4, token i)
+    const uint32_t *aq = reinterpret_cast<const uint32_t *>(xq) + (static_cast<size_t>(t0 + i) * 8 + s4 + 4 * g) * (BLOCKS ? 1 : 4);
+    const float *as = BLOCKS ? xs + static_cast<size_t>(s4) * ld + t0 + i : xs + static_cast<size_t>(t0) * 4 + lane;
+    const int as_slot = BLOCKS ? lane : 16 * (lane & 3) + (lane >> 2);
 
     u32x4_t bq[kSmallAhead];
     uint2 bs[kSmallAhead];
@@ -474,8 +502,14 @@ __global__ __launch_bounds__(256, 2) void q8_mmq_exact_small_kernel(Q8Matrix w, 
         const size_t b = static_cast<size_t>(cc) * ld;
 #pragma unroll
         for (int tt = 0; tt < TT; ++tt) {
-            at[slot][tt] = as[b * 4 + tt * 64];
-            av[slot][tt] = aq[b * 8 + tt * 128];
+            if constexpr (BLOCKS) {
+                at[slot][tt] = as[b * 4 + tt * 16];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) av[slot][tt][j] = aq[b * 32 + static_cast<size_t>(j) * ld * 8 + tt * 128];
+            } else {
+                at[slot][tt] = as[b * 4 + tt * 64];
+                av[slot][tt] = *reinterpret_cast<const u32x4_t *>(aq + b * 32 + tt * 512);
+            }
         }
         bq[slot] = wq[static_cast<size_t>(cc) * 64];
         bs[slot] = ws[static_cast<size_t>(cc) * 8];
@@ -488,7 +522,7 @@ __global__ __launch_bounds__(256, 2) void q8_mmq_exact_small_kernel(Q8Matrix w, 
     auto consume = [&](const u32x4_t &q4, const uint2 &sc, const u32x4_t (&a)[TT], const float (&asc)[TT]) {
         // the wave's own LDS, in order: no barrier
 #pragma unroll
-        for (int tt = 0; tt < TT; ++tt) scales[wave][tt][16 * (lane & 3) + (lane >> 2)] = asc[tt];
+        for (int tt = 0; tt < TT; ++tt) scales[wave][tt][as_slot] = asc[tt];
         wave_lds_fence();
         const f32x16 zero = {};
         f32x16 d = __builtin_amdgcn_mfma_f32_16x16x4f16(i8x4_to_h4(a[0][0]), i8x4_to_h4(q4[0]), zero, 0, 0, 0);
@@ -553,7 +587,7 @@ __global__ __launch_bounds__(256, 2) void q8_mmq_exact_small_kernel(Q8Matrix w, 
         }
 }
 
-// fortai_q8_quantize (fortai_q8_dot.c:153-198) of every token into X8: one
+// fortai_q8_quantize (fortai_q8_dot.c:153-198) of every token into block-major X8: one
 // thread per 4 values, 8 consecutive threads per block.
 __global__ __launch_bounds__(256) void q8_quantize_tokens_kernel(const float *__restrict__ x, int tokens, int width,
     int ld_x, int ld, int blocks_pad, int8_t *__restrict__ xq, float *__restrict__ xs) {
@@ -567,7 +601,8 @@ __global__ __launch_bounds__(256) void q8_quantize_tokens_kernel(const float *__
     uint16_t bits;
     const uint32_t packed = quantize_group(y, scale, bits);
     const int b = g >> 3, l = g & 7;
-    x8_store(xq, xs, ld, t, b, l, packed, scale);
+    reinterpret_cast<uint32_t *>(xq + (static_cast<size_t>(b) * ld + t) * 32)[l] = packed;
+    if (l == 0) xs[static_cast<size_t>(b) * ld + t] = scale;
 }
 
 }  // namespace
@@ -592,7 +627,7 @@ hipError_t launch_q8_quantize_tokens(const float *x, int tokens, int width, int 
 }
 
 hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, float *out, int ld_out,
-    const float *resid, hipStream_t stream) {
+    const float *resid, X8Layout layout, hipStream_t stream) {
     if (tokens <= 0 || ld_out < w.rows || w.rows <= 0) return hipErrorInvalidValue;
     const int ld = q8_tokens_ld(tokens);  // a multiple of the 64-token tile
     const int8_t *xq = static_cast<const int8_t *>(x8);
@@ -602,7 +637,8 @@ hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, fl
     // over rows 16 .. 9216, widths 1024 .. 9216 and 1 .. 1200 tokens: 64 x 64
     // tiles 2.15 while each CU has at most one, then 3.1 for two and 1.6 for
     // each more; 32 rows x 16 tokens 0.15 + 0.29 each, x 32 tokens 0.25 + 0.47
-    // each (a workgroup of either does 1/8 or 1/4 of the large one's work).
+    // each (a workgroup of either does 1/8 or 1/4 of the large one's work), and
+    // 0.05 + 0.85, 0.1 + 1.07 when block-major tokens crowd two L2 channels.
     constexpr int kCus = 256;
     auto per_cu = [&](int row_tile, int token_tile) {
         const long long wgs = static_cast<long long>((w.rows + row_tile - 1) / row_tile) * ((tokens + token_tile - 1) / token_tile);
@@ -610,18 +646,19 @@ hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, fl
     };
     const double nb = per_cu(kXTile, kXTile);
     const double large = nb <= 1.0 ? 2.15 : std::max(3.1, 1.6 * nb);
-    const double one = 0.15 + 0.29 * per_cu(kSmallRows, 16), two = 0.25 + 0.47 * per_cu(kSmallRows, 32);
+    const bool blocks = layout == X8Layout::BLOCKS;
+    const double one = (blocks ? 0.05 : 0.15) + (blocks ? 0.85 : 0.29) * per_cu(kSmallRows, 16);
+    const double two = (blocks ? 0.1 : 0.25) + (blocks ? 1.07 : 0.47) * per_cu(kSmallRows, 32);
     if (std::min(one, two) < large) {
         auto small = [&](auto tt_c) {
             constexpr int TT = decltype(tt_c)::value;
             const int tt_n = (tokens + 16 * TT - 1) / (16 * TT), rt_n = (w.rows + kSmallRows - 1) / kSmallRows;
             const dim3 sgrid((rt_n >= 8 ? (rt_n + 7) / 8 * 8 : rt_n) * tt_n);
-            if (resid)
-                hipLaunchKernelGGL((q8_mmq_exact_small_kernel<TT, 1>), sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld,
-                    out, ld_out, resid, tt_n);
-            else
-                hipLaunchKernelGGL((q8_mmq_exact_small_kernel<TT, 0>), sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld,
-                    out, ld_out, resid, tt_n);
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld, out, ld_out, resid, tt_n);
+            };
+            if (blocks) resid ? go(q8_mmq_exact_small_kernel<TT, 1, true>) : go(q8_mmq_exact_small_kernel<TT, 0, true>);
+            else resid ? go(q8_mmq_exact_small_kernel<TT, 1, false>) : go(q8_mmq_exact_small_kernel<TT, 0, false>);
             note_launch("q8_mmq_exact_small_kernel<%d,%s> grid %d", TT, resid ? "add" : "store", sgrid.x);
         };
         if (one <= two) small(std::integral_constant<int, 1>{});
@@ -629,33 +666,29 @@ hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, fl
         return hipGetLastError();
     }
     const size_t lds = 2 * sizeof(MmqExactStage);
-    if (resid)
-        hipLaunchKernelGGL((q8_mmq_exact_kernel<1>), grid, dim3(kXThreads), lds, stream, w, xq, xs, tokens, ld, out,
-            ld_out, resid);
-    else
-        hipLaunchKernelGGL((q8_mmq_exact_kernel<0>), grid, dim3(kXThreads), lds, stream, w, xq, xs, tokens, ld, out,
-            ld_out, resid);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kXThreads), lds, stream, w, xq, xs, tokens, ld, out, ld_out, resid);
+    };
+    if (blocks) resid ? go(q8_mmq_exact_kernel<1, true>) : go(q8_mmq_exact_kernel<0, true>);
+    else resid ? go(q8_mmq_exact_kernel<1, false>) : go(q8_mmq_exact_kernel<0, false>);
     note_launch("q8_mmq_exact_kernel<%s> grid %dx%d", resid ? "add" : "store", grid.x, grid.y);
     return hipGetLastError();
 }
 
 hipError_t launch_q8_mmq(const Q8Matrix &w, const void *x8, int tokens, float *out, int ld_out, const float *resid,
-    int32_t *dots, hipStream_t stream) {
-    if (tokens <= 0 || ld_out < w.rows || w.rows <= 0) return hipErrorInvalidValue;
+    int32_t *dots, X8Layout layout, hipStream_t stream) {
+    if (tokens <= 0 || ld_out < w.rows || w.rows <= 0 || (dots && layout != X8Layout::BLOCKS)) return hipErrorInvalidValue;
     const int ld = q8_tokens_ld(tokens);
     const int8_t *xq = static_cast<const int8_t *>(x8);
     const float *xs = reinterpret_cast<const float *>(xq + static_cast<size_t>(ld) * w.chunks * 4 * 32);
     const dim3 grid((w.rows + kRowTile - 1) / kRowTile, ld / kTokTile);
     const size_t lds = 2 * sizeof(MmqStage);
-    if (dots)
-        hipLaunchKernelGGL((q8_mmq_kernel<0, true>), grid, dim3(kMmqThreads), lds, stream, w, xq, xs, tokens, ld, out,
-            ld_out, resid, dots);
-    else if (resid)
-        hipLaunchKernelGGL((q8_mmq_kernel<1, false>), grid, dim3(kMmqThreads), lds, stream, w, xq, xs, tokens, ld, out,
-            ld_out, resid, dots);
-    else
-        hipLaunchKernelGGL((q8_mmq_kernel<0, false>), grid, dim3(kMmqThreads), lds, stream, w, xq, xs, tokens, ld, out,
-            ld_out, resid, dots);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, grid, dim3(kMmqThreads), lds, stream, w, xq, xs, tokens, ld, out, ld_out, resid, dots);
+    };
+    if (dots) go(q8_mmq_kernel<0, true, true>);
+    else if (layout == X8Layout::BLOCKS) resid ? go(q8_mmq_kernel<1, false, true>) : go(q8_mmq_kernel<0, false, true>);
+    else resid ? go(q8_mmq_kernel<1, false, false>) : go(q8_mmq_kernel<0, false, false>);
     note_launch("q8_mmq_kernel<%s> grid %dx%d", resid ? "add" : "store", grid.x, grid.y);
     return hipGetLastError();
 }
