@@ -50,7 +50,8 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kTokTile = 128;  // tokens per workgroup
 constexpr int kRowTile = 128;  // rows per workgroup
-constexpr int kMmqThreads = 256;
+constexpr int kRowTiles = 2;   // 32-row MFMA tiles per wave
+constexpr int kMmqThreads = 512;
 
 __device__ __forceinline__ v4i as_v4i(uint4 u) {
     v4i r;
@@ -76,15 +77,20 @@ struct MmqStage {
 
 __device__ __forceinline__ int half_slot(int n, int h) { return h ^ ((n >> 3) & 1); }
 
-// One workgroup: 128 tokens x 128 rows; wave w covers tokens 64 (w & 1) and
-// rows 64 (w >> 1) as 2 x 2 MFMA tiles of 32 x 32.  Chunk c + 1 is loaded
-// into registers while chunk c is consumed from LDS, then stored to the other
-// stage (one barrier per chunk).
+// One workgroup: 128 tokens x 128 rows, eight waves; a wave covers 32 tokens x
+// 64 rows (1 x 2 MFMA tiles of 32 x 32: a lane holds 16 tokens' scales, so one
+// token tile costs half the LDS scale reads of two).  The scale-and-accumulate
+// bounds it (48 vector instructions per MFMA), and 32 accumulators per lane
+// leave room for four waves per SIMD.  Chunk c + 1 is loaded into registers
+// while chunk c is consumed from LDS, then stored to the other stage (one
+// barrier per chunk).  With the quantizer, against four waves of 64 x 64 (two
+// per SIMD): 2560 x 9216 over 4096 tokens 486 -> 403 us, 9216 x 2560 over 4096
+// 322 -> 307 us, over 1200 121 -> 105 us, 3584 x 1024 over 700 29 -> 21 us.
 //   BLOCKS: X8 block-major, else chunk-major
 //   EPI 0: out[t * ld_out + row] = acc;  EPI 1: out = acc + resid (same index)
 //   DOTS: also write every int32 block dot to dots[(t * rows + row) * blocks + b]
 template <int EPI, bool DOTS, bool BLOCKS>
-__global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
+__global__ __launch_bounds__(kMmqThreads, 4) void q8_mmq_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
     const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
     const float *__restrict__ resid, int32_t *__restrict__ dots) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -94,20 +100,21 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
     const int i = lane & 31, h = lane >> 5;
     const int t0 = static_cast<int>(blockIdx.y) * kTokTile;
     const int r0 = static_cast<int>(blockIdx.x) * kRowTile;
-    const int twl = (wave & 1) * 64;   // wave's first token within the tile
-    const int rwl = (wave >> 1) * 64;  // wave's first row within the tile
+    const int twl = (wave & 3) * 32;               // wave's first token within the tile
+    const int rwl = (wave >> 2) * 32 * kRowTiles;  // wave's first row within the tile
     const int chunks = w.chunks;
     // global sources of this thread's share of a chunk:
     //  tokens: 128 tokens x 8 lane parts (BLOCKS: 4 blocks x 128 tokens x 2 halves) = 1024 pieces, 4 per thread
     //  rows:   16 row groups x 64 lanes          = 1024 pieces, 4 per thread
     //  token scales: 512 floats, 2 per thread;  row scales: 128 x uint2, threads < 128
     const int g_last = w.row_groups - 1;
-    u32x4_t ra[4], rb[4];  // plain vectors (arrays of the uint4 class stay in scratch)
-    float rs[2];
+    constexpr int kPieces = 1024 / kMmqThreads, kScales = 512 / kMmqThreads;
+    u32x4_t ra[kPieces], rb[kPieces];  // plain vectors (arrays of the uint4 class stay in scratch)
+    float rs[kScales];
     uint2 rws = make_uint2(0u, 0u);
     auto fetch = [&](int c) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < kPieces; ++k) {
             const int p = tid + k * kMmqThreads;          // 0..1023
             if constexpr (BLOCKS)  // block p / 256, token p / 2 % 128, half p % 2
                 ra[k] = *reinterpret_cast<const u32x4_t *>(xq + (static_cast<size_t>(4 * c + (p >> 8)) * ld + t0) * 32 + (p & 255) * 16);
@@ -118,7 +125,7 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
             rb[k] = reinterpret_cast<const u32x4_t *>(w.quants)[(static_cast<size_t>(g) * chunks + c) * 64 + (p & 63)];
         }
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
+        for (int k = 0; k < kScales; ++k) {
             const int p = tid + k * kMmqThreads;  // 0..511: token p / 4, block p % 4 (BLOCKS: block p / 128, token p % 128)
             rs[k] = BLOCKS ? xs[static_cast<size_t>(4 * c + (p >> 7)) * ld + t0 + (p & 127)]
                            : xs[(static_cast<size_t>(c) * ld + t0) * 4 + p];
@@ -132,7 +139,7 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
         // piece p: token or row p / 8, bytes 4l..4l+3 (l = p % 8) of the four blocks
         uint32_t *da = reinterpret_cast<uint32_t *>(&st.a[0][0][0]), *db = reinterpret_cast<uint32_t *>(&st.b[0][0][0]);
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < kPieces; ++k) {
             const int p = tid + k * kMmqThreads;
             const int n = p >> 3, l = p & 7;
             const int base = (n * 2 + half_slot(n, l >> 2)) * 4 + (l & 3);
@@ -145,7 +152,7 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
             }
         }
 #pragma unroll
-        for (int k = 0; k < 2; ++k) {
+        for (int k = 0; k < kScales; ++k) {
             const int p = tid + k * kMmqThreads;
             if constexpr (BLOCKS) st.as[p >> 7][p & 127] = rs[k];
             else st.as[p & 3][p >> 2] = rs[k];
@@ -158,13 +165,11 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
         }
     };
 
-    float acc[2][2][16];
+    float acc[kRowTiles][16];
 #pragma unroll
-    for (int ta = 0; ta < 2; ++ta)
+    for (int f = 0; f < kRowTiles; ++f)
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[ta][f][v] = 0.0f;
+        for (int v = 0; v < 16; ++v) acc[f][v] = 0.0f;
 
     fetch(0);
     stash(stage[0]);
@@ -176,47 +181,41 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
         // the chunk and spills)
 #pragma unroll 1
         for (int j = 0; j < 4; ++j) {
-            uint4 af[2], bf[2];
-            float wsc[2];
+            const int t = twl + i;
+            const v4i af = as_v4i(st.a[j][t][half_slot(t, h)]);
+            // this lane's 16 tokens: twl + 8 (v / 4) + 4 h + v % 4
+            float tsc[16];
+            const float4 *s4 = reinterpret_cast<const float4 *>(&st.as[j][twl + 4 * h]);
 #pragma unroll
-            for (int ta = 0; ta < 2; ++ta) {
-                const int t = twl + 32 * ta + i;
-                af[ta] = st.a[j][t][half_slot(t, h)];
+            for (int q = 0; q < 4; ++q) {
+                const float4 s = s4[2 * q];
+                tsc[4 * q] = s.x; tsc[4 * q + 1] = s.y; tsc[4 * q + 2] = s.z; tsc[4 * q + 3] = s.w;
             }
+            v4i bf[kRowTiles];
+            float wsc[kRowTiles];
 #pragma unroll
-            for (int f = 0; f < 2; ++f) {
+            for (int f = 0; f < kRowTiles; ++f) {
                 const int row = rwl + 32 * f + i;
-                bf[f] = st.b[j][row][half_slot(row, h)];
+                bf[f] = as_v4i(st.b[j][row][half_slot(row, h)]);
                 wsc[f] = st.bs[j][row];
             }
 #pragma unroll
-            for (int ta = 0; ta < 2; ++ta) {
-                // this lane's 16 tokens: twl + 32 ta + 8 (v / 4) + 4 h + v % 4
-                float tsc[16];
-                const float4 *s4 = reinterpret_cast<const float4 *>(&st.as[j][twl + 32 * ta + 4 * h]);
+            for (int f = 0; f < kRowTiles; ++f) {
+                const v16i zero = {};
+                const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(af, bf[f], zero, 0, 0, 0);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const float4 s = s4[2 * q];
-                    tsc[4 * q] = s.x; tsc[4 * q + 1] = s.y; tsc[4 * q + 2] = s.z; tsc[4 * q + 3] = s.w;
-                }
+                for (int v = 0; v < 16; ++v)
+                    acc[f][v] = __builtin_fmaf(wsc[f] * tsc[v], static_cast<float>(d[v]), acc[f][v]);
+                // keep one MFMA result live at a time (the other waves of the
+                // SIMD cover the MFMA latency)
+                __builtin_amdgcn_sched_barrier(0);
+                if constexpr (DOTS) {
+                    const int row = r0 + rwl + 32 * f + i, blk = 4 * c + j;
+                    if (row < w.rows && blk < w.blocks) {
 #pragma unroll
-                for (int f = 0; f < 2; ++f) {
-                    const v16i zero = {};
-                    const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(as_v4i(af[ta]), as_v4i(bf[f]), zero, 0, 0, 0);
-#pragma unroll
-                    for (int v = 0; v < 16; ++v)
-                        acc[ta][f][v] = __builtin_fmaf(wsc[f] * tsc[v], static_cast<float>(d[v]), acc[ta][f][v]);
-                    // keep one MFMA result live at a time (the other wave of
-                    // the SIMD covers the MFMA latency)
-                    __builtin_amdgcn_sched_barrier(0);
-                    if constexpr (DOTS) {
-                        const int row = r0 + rwl + 32 * f + i, blk = 4 * c + j;
-                        if (row < w.rows && blk < w.blocks) {
-#pragma unroll
-                            for (int v = 0; v < 16; ++v) {
-                                const int t = t0 + twl + 32 * ta + 8 * (v >> 2) + 4 * h + (v & 3);
-                                if (t < tokens) dots[(static_cast<size_t>(t) * w.rows + row) * w.blocks + blk] = d[v];
-                            }
+                        for (int v = 0; v < 16; ++v) {
+                            const int tt = t0 + twl + 8 * (v >> 2) + 4 * h + (v & 3);
+                            if (tt < tokens) dots[(static_cast<size_t>(tt) * w.rows + row) * w.blocks + blk] = d[v];
                         }
                     }
                 }
@@ -226,20 +225,120 @@ __global__ __launch_bounds__(kMmqThreads, 2) void q8_mmq_kernel(Q8Matrix w, cons
         __syncthreads();
     }
 #pragma unroll
-    for (int ta = 0; ta < 2; ++ta) {
+    for (int f = 0; f < kRowTiles; ++f) {
+        const int row = r0 + rwl + 32 * f + i;
+        if (row >= w.rows) continue;
 #pragma unroll
-        for (int f = 0; f < 2; ++f) {
-            const int row = r0 + rwl + 32 * f + i;
-            if (row >= w.rows) continue;
+        for (int v = 0; v < 16; ++v) {
+            const int t = t0 + twl + 8 * (v >> 2) + 4 * h + (v & 3);
+            if (t >= tokens) continue;
+            const size_t o = static_cast<size_t>(t) * ld_out + row;
+            if constexpr (EPI == 1) out[o] = acc[f][v] + resid[o];
+            else out[o] = acc[f][v];
+        }
+    }
+}
+
+// The same product for few tokens or few rows, where 128 x 128 tiles leave most
+// CUs idle: a wave takes 32 rows x 32 tokens, one MFMA per block, with no LDS
+// but the token scales: the four 16-byte pieces that hold lane parts
+// 4 h .. 4 h + 3 of row (or chunk-major token) i for four blocks are the
+// operands of the chunk's four instructions as they are.  The four waves of a
+// workgroup share the tokens.  Operands are loaded two chunks ahead.  With the
+// quantizer, 128 x 128 tiles before: 9216 x 2560, 77 tokens 57 -> 21 us;
+// 2560 x 9216, 301 tokens 192 -> 63 us; 32 x 2560, 2103 tokens 61 -> 24 us.
+constexpr int kFewRows = 128, kFewTokens = 32;
+constexpr int kCus = 256;  // compute units (the launches' tile rules)
+
+template <int EPI, bool BLOCKS>
+__global__ __launch_bounds__(256, 2) void q8_mmq_few_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
+    const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
+    const float *__restrict__ resid, int token_tiles) {
+    __shared__ __align__(16) float scales[4][4][kFewTokens];  // per wave: a chunk's token scales [block][token]
+    const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
+    const int i = lane & 31, h = lane >> 5;
+    // XCD-grouped as q8_mmq_exact_small_kernel's workgroups
+    const int id = static_cast<int>(blockIdx.x);
+    const bool grouped = w.rows > 7 * kFewRows;
+    const int row_tile = grouped ? id / 8 / token_tiles * 8 + id % 8 : id / token_tiles;
+    const int t0 = (grouped ? id / 8 % token_tiles : id % token_tiles) * kFewTokens;
+    const int row = row_tile * kFewRows + 32 * wave + i;
+    if (row - i >= w.rows) return;  // no row of this wave (no barrier follows)
+    const int chunks = w.chunks;
+    const int g8 = min(row >> 3, w.row_groups - 1);  // clamped; rows past the end are not stored
+    const u32x4_t *wq = reinterpret_cast<const u32x4_t *>(w.quants) + static_cast<size_t>(g8) * chunks * 64 + (row & 7) * 8 + 4 * h;
+    const uint2 *ws = w.scales + static_cast<size_t>(g8) * chunks * 8 + (row & 7);
+    const u32x4_t *aq = reinterpret_cast<const u32x4_t *>(xq) + (BLOCKS ? static_cast<size_t>(t0 + i) * 2 + h : static_cast<size_t>(t0 + i) * 8 + 4 * h);
+    // scale word k of this lane: token lane / 4 + 16 k, block lane % 4 (BLOCKS: block h + 2 k, token i)
+    const float *as = BLOCKS ? xs + static_cast<size_t>(h) * ld + t0 + i : xs + static_cast<size_t>(t0) * 4 + lane;
+    float *sc = &scales[wave][0][0];
+    const int slot = BLOCKS ? lane : (lane & 3) * kFewTokens + (lane >> 2);
+
+    u32x4_t bq[2][4], av[2][4];
+    uint2 bs[2];
+    float at[2][2];
+    auto fetch = [&](int c, int s) {
+        const size_t cc = static_cast<size_t>(min(c, chunks - 1));
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int t = t0 + twl + 32 * ta + 8 * (v >> 2) + 4 * h + (v & 3);
-                if (t >= tokens) continue;
-                const size_t o = static_cast<size_t>(t) * ld_out + row;
-                if constexpr (EPI == 1) out[o] = acc[ta][f][v] + resid[o];
-                else out[o] = acc[ta][f][v];
+        for (int k = 0; k < 2; ++k) at[s][k] = as[cc * 4 * ld + (BLOCKS ? static_cast<size_t>(2 * k) * ld : 64 * k)];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            av[s][k] = BLOCKS ? aq[(cc * 4 + k) * ld * 2] : aq[cc * ld * 8 + k];
+            bq[s][k] = wq[cc * 64 + k];
+        }
+        bs[s] = ws[cc * 8];
+    };
+    float acc[16];
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.0f;
+    auto operand = [](const u32x4_t (&p)[4], int j) {
+        return v4i{static_cast<int>(p[0][j]), static_cast<int>(p[1][j]), static_cast<int>(p[2][j]), static_cast<int>(p[3][j])};
+    };
+    auto consume = [&](int s) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) sc[slot + (BLOCKS ? 64 : 16) * k] = at[s][k];
+        wave_lds_fence();
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const v4i a = BLOCKS ? v4i{static_cast<int>(av[s][j].x), static_cast<int>(av[s][j].y), static_cast<int>(av[s][j].z),
+                static_cast<int>(av[s][j].w)} : operand(av[s], j);
+            const v16i zero = {};
+            const v16i d = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, operand(bq[s], j), zero, 0, 0, 0);
+            const uint32_t sh = j < 2 ? bs[s].x : bs[s].y;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const float4 x = *reinterpret_cast<const float4 *>(sc + j * kFewTokens + 8 * q + 4 * h);
+                const float xv[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float p = j & 1 ? half_times<true>(sh, xv[u]) : half_times<false>(sh, xv[u]);
+                    acc[4 * q + u] = __builtin_fmaf(p, static_cast<float>(d[4 * q + u]), acc[4 * q + u]);
+                }
             }
         }
+        wave_lds_fence();
+    };
+    fetch(0, 0);
+    fetch(1, 1);
+    int c = 0;
+    for (; c + 2 <= chunks; c += 2) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k) {
+            __builtin_amdgcn_sched_barrier(0);
+            consume(k);
+            __builtin_amdgcn_sched_barrier(0);
+            fetch(c + k + 2, k);
+        }
+    }
+    if (c < chunks) consume(0);
+    if (row >= w.rows) return;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int t = t0 + 8 * (v >> 2) + 4 * h + (v & 3);
+        if (t >= tokens) continue;
+        const size_t o = static_cast<size_t>(t) * ld_out + row;
+        if constexpr (EPI == 1) out[o] = acc[v] + resid[o];
+        else out[o] = acc[v];
     }
 }
 
@@ -639,7 +738,6 @@ hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, fl
     // each more; 32 rows x 16 tokens 0.15 + 0.29 each, x 32 tokens 0.25 + 0.47
     // each (a workgroup of either does 1/8 or 1/4 of the large one's work), and
     // 0.05 + 0.85, 0.1 + 1.07 when block-major tokens crowd two L2 channels.
-    constexpr int kCus = 256;
     auto per_cu = [&](int row_tile, int token_tile) {
         const long long wgs = static_cast<long long>((w.rows + row_tile - 1) / row_tile) * ((tokens + token_tile - 1) / token_tile);
         return static_cast<double>((wgs + kCus - 1) / kCus);
@@ -681,6 +779,25 @@ hipError_t launch_q8_mmq(const Q8Matrix &w, const void *x8, int tokens, float *o
     const int ld = q8_tokens_ld(tokens);
     const int8_t *xq = static_cast<const int8_t *>(x8);
     const float *xs = reinterpret_cast<const float *>(xq + static_cast<size_t>(ld) * w.chunks * 4 * 32);
+    // Time per chunk by workgroups per CU, us, measured as for the exact
+    // product: 128 x 128 tiles 1.75 while each CU has at most one, then 1.65
+    // each; 128 rows x 32 tokens (a quarter of the work) 0.2 + 0.66 each.
+    auto per_cu = [&](int row_tile, int token_tile) {
+        const long long wgs = static_cast<long long>((w.rows + row_tile - 1) / row_tile) * ((tokens + token_tile - 1) / token_tile);
+        return static_cast<double>((wgs + kCus - 1) / kCus);
+    };
+    const double nl = per_cu(kRowTile, kTokTile);
+    if (!dots && 0.2 + 0.66 * per_cu(kFewRows, kFewTokens) < (nl <= 1.0 ? 1.75 : 1.65 * nl)) {
+        const int tt_n = (tokens + kFewTokens - 1) / kFewTokens, rt_n = (w.rows + kFewRows - 1) / kFewRows;
+        const dim3 sgrid((rt_n >= 8 ? (rt_n + 7) / 8 * 8 : rt_n) * tt_n);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld, out, ld_out, resid, tt_n);
+        };
+        if (layout == X8Layout::BLOCKS) resid ? go(q8_mmq_few_kernel<1, true>) : go(q8_mmq_few_kernel<0, true>);
+        else resid ? go(q8_mmq_few_kernel<1, false>) : go(q8_mmq_few_kernel<0, false>);
+        note_launch("q8_mmq_few_kernel<%s> grid %d", resid ? "add" : "store", sgrid.x);
+        return hipGetLastError();
+    }
     const dim3 grid((w.rows + kRowTile - 1) / kRowTile, ld / kTokTile);
     const size_t lds = 2 * sizeof(MmqStage);
     auto go = [&](auto kernel) {

@@ -164,3 +164,43 @@ def test_mmq_lane_order_tiles(ctx, rows, width, tokens):
     for b in (dx, dq, out, want):
         b.free()
     W.free()
+
+
+@pytest.mark.parametrize("rows,width,tokens", [(1, 32, 1), (31, 96, 33), (130, 160, 64), (897, 288, 31), (1030, 1056, 40),
+                                               (2560, 544, 700), (128, 2560, 129), (4100, 128, 520)])
+def test_mmq_tiles(ctx, oracle, rows, width, tokens):
+    """The whole-block product's tile choices (128 x 128 and 128 rows x 32
+    tokens, fewer and more than eight row tiles, odd chunk counts): every output
+    is the scalar reference's block-order sum acc = fma(w_scale * x_scale,
+    dot, acc) of exact int32 block dots, bit for bit on a sample of tokens; the
+    residual is added in place."""
+    rng = np.random.default_rng(rows + 5 * width + tokens)
+    w = synth.q8_blocks(rng, rows, width)
+    nb = width // 32
+    W = B.Q8Weights(ctx, w, rows, width)
+    x = rng.standard_normal((tokens, width)).astype(np.float32)
+    x[0, :32] = 0.0
+    dx = ctx.upload_array(x)
+    dq = ctx.alloc(B.load().fortai_hip_q8_tokens_bytes(tokens, width))
+    out = ctx.alloc(tokens * rows * 4)
+    ctx.call("fortai_hip_q8_quantize_tokens_device", ctx.h, dx.ptr, tokens, width, dq.ptr)
+    ctx.call("fortai_hip_q8_mmq_device", ctx.h, W.h, dq.ptr, tokens, out.ptr, None, None)
+    got = out.download(np.float32).reshape(tokens, rows)
+    ws = w.reshape(rows, nb, 34)[:, :, :2].copy().view(np.float16).reshape(rows, nb).astype(np.float32)
+    for t in sorted({0, 1 % tokens, 31 % tokens, 32 % tokens, tokens // 2, tokens - 1}):
+        qr, sr = oracle.quantize(x[t])
+        dots = oracle.block_dots(w, qr, rows, nb).astype(np.float64)
+        acc = np.zeros(rows, np.float32)
+        for b in range(nb):
+            # a float64 product and sum of a 24-bit and a 20-bit factor and a
+            # float32 is exact here up to its one rounding to float32, unless
+            # the float64 sum itself rounds: allow that double rounding one ulp
+            acc = ((ws[:, b] * np.float32(sr[b])).astype(np.float64) * dots[:, b] + acc).astype(np.float32)
+        assert rel_err(got[t], acc) <= 2.0 ** -22, f"token {t}"
+    resid = rng.standard_normal((tokens, rows)).astype(np.float32)
+    out.upload(resid)
+    ctx.call("fortai_hip_q8_mmq_device", ctx.h, W.h, dq.ptr, tokens, out.ptr, out.ptr, None)
+    assert np.array_equal(out.download(np.float32).reshape(tokens, rows), (got + resid).astype(np.float32))
+    for b in (dx, dq, out):
+        b.free()
+    W.free()
