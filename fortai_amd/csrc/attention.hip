@@ -3,9 +3,11 @@
 // its summation orders kept (attention_exact.h), so the output is
 // bit-identical to the CPU path (fortai_qwen35_cpu.f90:990-1033).
 //
-// Two kernels: scores (one workgroup per kv head x 64 positions; the one
-// that holds the new position also appends it) and output (one workgroup per
-// head x 8 value dims: softmax weights, the P.V chains and the sigmoid gate).
+// Three kernels: scores (one workgroup per kv head x 64 positions; the one
+// that holds the new position also appends it), softmax (e values and Z tables)
+// and output (one workgroup per head x 8 value dims: the P.V chains and the
+// sigmoid gate).  Beyond exact_max positions the first also sums its values
+// (flash-decoding) and the last merges the blocks.
 #include "attention_exact.h"
 #include "fortai_hip_internal.h"
 #include "fortai_hip_kernels.h"
@@ -22,8 +24,6 @@ constexpr int kLoads = ea::kPosBlock * (kMaxHead / 8) / ea::kThreads;
 constexpr int kQLoads = kMaxGroup * kMaxHead / ea::kThreads;
 
 typedef uint32_t v4u __attribute__((ext_vector_type(4)));
-
-constexpr int kChunk = 256;  // positions per split-K chunk (long contexts)
 
 // The per-sequence workspace behind AttentionParams::partial, in floats:
 //   scores [heads][max_context] | e values [heads][max_context] |
@@ -51,7 +51,6 @@ __device__ __forceinline__ float *ztab_of(const AttentionParams &p) {
 // Sequence s of a batch (blockIdx.y): every per-sequence buffer is laid out
 // [batch][...] with the single-sequence size, and position[s] is its own.
 __device__ __forceinline__ AttentionParams attention_seq(AttentionParams p, int s) {
-    const size_t nmax = (static_cast<size_t>(p.max_context) + kChunk - 1) / kChunk;
     p.q += static_cast<size_t>(s) * p.heads * 2 * p.head;
     p.k += static_cast<size_t>(s) * p.kv_heads * p.head;
     p.v += static_cast<size_t>(s) * p.kv_heads * p.value;
@@ -62,7 +61,7 @@ __device__ __forceinline__ AttentionParams attention_seq(AttentionParams p, int 
     p.out += static_cast<size_t>(s) * p.heads * p.value;
     if (p.out_q8l) p.out_q8l = static_cast<unsigned char *>(p.out_q8l) + static_cast<size_t>(s) * q8l_bytes(p.heads * p.value);
     p.position += s;
-    if (p.split) p.split += static_cast<size_t>(s) * p.heads * nmax * (p.value + 2);
+    if (p.split) p.split += static_cast<size_t>(s) * p.heads * score_blocks(p.max_context) * p.value;
     return p;
 }
 
@@ -88,19 +87,80 @@ __device__ __forceinline__ void out_quantize64(const AttentionParams &p, int h, 
     }
 }
 
-__global__ __launch_bounds__(ea::kThreads) void attention_scores_kernel(const AttentionParams p_batch) {
-    FORTAI_TRACE_SCOPE(3);
-    const AttentionParams p = attention_seq(p_batch, static_cast<int>(blockIdx.y));
-    __shared__ __align__(16) float qh[kMaxGroup * kMaxHead];
-    __shared__ __align__(16) float kn[kMaxHead];
-    __shared__ __align__(16) float2 rs[kMaxHead / 2];
-    __shared__ __align__(16) uint16_t ktile[ea::kPosBlock][kMaxHead + 8];
-    __shared__ int overflow;
+struct ScoresLds {
+    float qh[kMaxGroup * kMaxHead];  // normalized q of the group's heads; SPLIT: then e[head][position]
+    float kn[kMaxHead];
+    float2 rs[kMaxHead / 2];
+    uint16_t ktile[ea::kPosBlock][kMaxHead + 8];  // SPLIT: then the position groups' value sums
+    int overflow;
+};
+
+// Value pieces of a split block: thread t takes dims 8 (t % 32) .. + 7 of
+// positions 8 (t / 32) .. + 7.
+constexpr int kSplitSlices = kMaxHead / 8;
+constexpr int kSplitGroups = ea::kThreads / kSplitSlices;
+constexpr int kSplitPer = ea::kPosBlock / kSplitGroups;  // positions per thread
+static_assert(kSplitPer % 4 == 0, "whole float4 reads of e");
+static_assert(kMaxGroup * kSplitGroups * kMaxHead * sizeof(float) <= sizeof(ScoresLds::ktile), "the value sums fit the key tile");
+
+template <bool FINITE>
+__device__ __forceinline__ void split_values(const AttentionParams &p, const uint4 (&vv)[kSplitPer], int n, int group,
+    ScoresLds &L, float *dst, size_t head_stride) {
+    const int tid = static_cast<int>(threadIdx.x), slice = tid % kSplitSlices, pg = tid / kSplitSlices;
+    float acc[kMaxGroup][8];
+#pragma unroll
+    for (int g = 0; g < kMaxGroup; ++g)
+#pragma unroll
+        for (int d = 0; d < 8; ++d) acc[g][d] = 0.0f;
+#pragma unroll
+    for (int i0 = 0; i0 < kSplitPer; i0 += 4) {
+        float e[kMaxGroup][4];
+#pragma unroll
+        for (int g = 0; g < kMaxGroup; ++g) {
+            const float4 e4 = *reinterpret_cast<const float4 *>(L.qh + g * ea::kPosBlock + pg * kSplitPer + i0);
+            e[g][0] = e4.x; e[g][1] = e4.y; e[g][2] = e4.z; e[g][3] = e4.w;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if (pg * kSplitPer + i0 + i >= n) continue;  // (a clamped copy of the last position)
+            const uint32_t hw[4] = {vv[i0 + i].x, vv[i0 + i].y, vv[i0 + i].z, vv[i0 + i].w};
+#pragma unroll
+            for (int d = 0; d < 8; ++d) {
+                const float v = ea::kv<FINITE>(static_cast<uint16_t>(hw[d >> 1] >> (16 * (d & 1))));
+#pragma unroll
+                for (int g = 0; g < kMaxGroup; ++g) acc[g][d] = __builtin_fmaf(e[g][i], v, acc[g][d]);
+            }
+        }
+    }
+    float *part = reinterpret_cast<float *>(&L.ktile[0][0]);  // [head][position group][dim]
+#pragma unroll
+    for (int g = 0; g < kMaxGroup; ++g) {
+        float4 *o = reinterpret_cast<float4 *>(part + (g * kSplitGroups + pg) * kMaxHead + slice * 8);
+        o[0] = make_float4(acc[g][0], acc[g][1], acc[g][2], acc[g][3]);
+        o[1] = make_float4(acc[g][4], acc[g][5], acc[g][6], acc[g][7]);
+    }
+    __syncthreads();
+    if (tid >= p.value) return;
+    for (int g = 0; g < group; ++g) {
+        float o = 0.0f;
+#pragma unroll
+        for (int k = 0; k < kSplitGroups; ++k) o += part[(g * kSplitGroups + k) * kMaxHead + tid];
+        dst[g * head_stride + tid] = o;
+    }
+}
+
+// One block of kPosBlock positions of one kv head, for its GQA group.
+// SPLIT (beyond exact_max): instead of the scores, the block's max m_b, sum
+// Z_b of exp(s - m_b) and value sums o_b = sum exp(s - m_b) v, which merge_block
+// combines (flash-decoding).
+template <bool SPLIT>
+__device__ __forceinline__ void scores_block(const AttentionParams &p, int pos, ScoresLds &L) {
+    float *qh = L.qh, *kn = L.kn;
+    float2 *rs = L.rs;
+    auto &ktile = L.ktile;
+    int &overflow = L.overflow;
     const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6, lane = tid & 63;
-    FORTAI_ATT_MARK(16);
-    const int pos = *p.position;
-    if (pos < 0 || pos >= p.max_context) return;  // never index past the cache
-    const int positions = pos + 1, nblk_max = (p.max_context + ea::kPosBlock - 1) / ea::kPosBlock;
+    const int positions = pos + 1;
     // block-major: the blocks that hold positions are dispatched first, the
     // ones past the current position (which only read it and exit) last
     const int b = div(static_cast<int>(blockIdx.x), p.div_kv_heads);
@@ -163,6 +223,16 @@ __global__ __launch_bounds__(ea::kThreads) void attention_scores_kernel(const At
         const int j = div(li, p.div_segs), sg = li - j * static_cast<int>(p.div_segs.d);
         if (j < n) *reinterpret_cast<v4u *>(&ktile[j][sg * 8]) = kr[i];
     }
+    // the block's values, while the scores are formed (the keys' registers are free)
+    const int vslice = tid % kSplitSlices, vpg = tid / kSplitSlices;
+    const int vd0 = (vslice * 8 < VD ? vslice : 0) * 8;  // slices past VD repeat slice 0 and are not stored
+    uint4 vv[SPLIT ? kSplitPer : 1];
+    if constexpr (SPLIT) {
+#pragma unroll
+        for (int i = 0; i < kSplitPer; ++i)
+            vv[i] = *reinterpret_cast<const uint4 *>(
+                p.vcache + (static_cast<size_t>(p0 + min(vpg * kSplitPer + i, n - 1)) * NKV + kvh) * VD + vd0);
+    }
     __syncthreads();
     FORTAI_ATT_MARK(19);
     if (owns_new) {
@@ -184,26 +254,152 @@ __global__ __launch_bounds__(ea::kThreads) void attention_scores_kernel(const At
     const bool finite = flag == 0 && overflow == 0;
     const float sqrt_head = sqrtf(static_cast<float>(HD));
     const int gi = tid >> 6, j = tid & 63;
+    float ev = 0.0f;  // SPLIT: exp(s - m_b)
     if (gi < group) {  // wave gi: head kvh * group + gi, positions p0 + lane
         constexpr float kLowest = -3.402823466e38f;  // -huge(1.0_real32)
         float sc = kLowest;
         if (j < n) {
             const float *qg = qh + gi * HD;
             const uint16_t *kr = &ktile[j][0];
-            if (finite) sc = HD == 256 ? ea::score_n<true, 256>(qg, kr, sqrt_head) : ea::score<true>(qg, kr, HD, sqrt_head);
+            if (finite) sc = !SPLIT && HD == 256 ? ea::score_n<true, 256>(qg, kr, sqrt_head) : ea::score<true>(qg, kr, HD, sqrt_head);
             else sc = ea::score<false>(qg, kr, HD, sqrt_head);
-            p.partial[static_cast<size_t>(kvh * group + gi) * p.max_context + p0 + j] = sc;
+            if constexpr (!SPLIT) p.partial[static_cast<size_t>(kvh * group + gi) * p.max_context + p0 + j] = sc;
         }
-        // the block's max and sum of exp(s - max) (a fast exp, in double): the
-        // softmax kernel's estimates start from these, not from every score
         const float mb = wave_max(sc);
-        double t = j < n ? static_cast<double>(__expf(sc - mb)) : 0.0;
-        t = wave_sum(t);
-        if (j == 0)
-            block_stats_of(p)[static_cast<size_t>(kvh * group + gi) * score_blocks(p.max_context) + b] =
-                make_float2(mb, static_cast<float>(t));
+        float2 *stats = block_stats_of(p) + static_cast<size_t>(kvh * group + gi) * score_blocks(p.max_context) + b;
+        if constexpr (SPLIT) {
+            ev = j < n ? expf_libm(sc - mb) : 0.0f;
+            const float z = wave_sum(ev);
+            if (j == 0) *stats = make_float2(mb, z);
+        } else {
+            // the block's max and sum of exp(s - max) (a fast exp, in double): the
+            // softmax kernel's estimates start from these, not from every score
+            double t = j < n ? static_cast<double>(__expf(sc - mb)) : 0.0;
+            t = wave_sum(t);
+            if (j == 0) *stats = make_float2(mb, static_cast<float>(t));
+        }
     }
     FORTAI_ATT_MARK(20);
+    if constexpr (SPLIT) {
+        // the new position's values come from the projection, not from the cache
+        if (owns_new) {
+            const float *vn = p.v + static_cast<size_t>(kvh) * VD + vd0;
+#pragma unroll
+            for (int i = 0; i < kSplitPer; ++i) {
+                if (p0 + vpg * kSplitPer + i < pos) continue;  // at pos, and the clamped copies of it
+                uint32_t w[4];
+#pragma unroll
+                for (int d = 0; d < 4; ++d)
+                    w[d] = float_to_half_kv(vn[2 * d]) | static_cast<uint32_t>(float_to_half_kv(vn[2 * d + 1])) << 16;
+                vv[i] = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+        __syncthreads();  // every wave is done with qh and the key tile
+        qh[tid] = ev;     // [head][position]; 0 past n and past the group
+        __syncthreads();
+        const size_t head_stride = static_cast<size_t>(score_blocks(p.max_context)) * VD;
+        float *dst = p.split + static_cast<size_t>(kvh * group) * head_stride + static_cast<size_t>(b) * VD;
+        if (finite) split_values<true>(p, vv, n, group, L, dst, head_stride);
+        else split_values<false>(p, vv, n, group, L, dst, head_stride);
+    }
+}
+
+__global__ __launch_bounds__(ea::kThreads) void attention_scores_kernel(const AttentionParams p_batch) {
+    FORTAI_TRACE_SCOPE(3);
+    const AttentionParams p = attention_seq(p_batch, static_cast<int>(blockIdx.y));
+    __shared__ __align__(16) ScoresLds L;
+    FORTAI_ATT_MARK(16);
+    const int pos = *p.position;
+    if (pos < 0 || pos >= p.max_context) return;  // never index past the cache
+    scores_block<false>(p, pos, L);
+}
+
+// The first kernel of contexts longer than exact_max: the scores up to it,
+// scores and values in one pass beyond.  Bound by latency: position, q norm, key
+// block, the 256 dependent adds of a score, values; four 40 KB workgroups share
+// a CU and cover each other's waits (1024 of them, 32768 positions of two kv
+// heads, are one round).  So its registers are held to four waves per SIMD, the
+// values are loaded into the keys' registers, and the scores run in the rolled
+// form (unrolled, at three waves per SIMD: 24 against 21-22 us).  A pass over
+// the scores with the values, 256 positions per workgroup, and the merge were
+// launches of their own before: 8 heads, 32768 positions, whole call 38.3 ->
+// 28.7 us (67 MB: 2.3 TB/s).
+__global__ __launch_bounds__(ea::kThreads, 4) void attention_split_kernel(const AttentionParams p_batch) {
+    const AttentionParams p = attention_seq(p_batch, static_cast<int>(blockIdx.y));
+    __shared__ __align__(16) ScoresLds L;
+    const int pos = *p.position;
+    if (pos < 0 || pos >= p.max_context) return;
+    if (pos + 1 > p.exact_max) scores_block<true>(p, pos, L);
+    else scores_block<false>(p, pos, L);
+}
+
+// Beyond exact_max, DIMS value dims of head h from the blocks' partials:
+// M = max m_b, Z = sum Z_b e^(m_b - M), out = (sum o_b e^(m_b - M)) / Z *
+// sigmoid(gate).  Blocks go to kMergeParts running sums per dim (block b to sum
+// b % kMergeParts), whatever DIMS is, so that every output kernel gives the same
+// bits.  lds: kMergeTile + kMergeParts * DIMS + 4 floats.
+constexpr int kMaxSplitPositions = 1 << 20;
+constexpr int kMergeTile = 1024;
+constexpr int kMergeParts = 32;
+template <int DIMS>
+__device__ __forceinline__ void merge_block(const AttentionParams &p, int h, int d0, int positions, float *lds) {
+    constexpr int kThreadsPerDim = ea::kThreads / DIMS, kSums = kMergeParts / kThreadsPerDim;
+    static_assert(kSums * kThreadsPerDim == kMergeParts, "whole sums per thread");
+    constexpr int kAhead = 16 / (kSums > 4 ? 4 : kSums);  // blocks in flight per sum
+    float *f = lds, *part = lds + kMergeTile, *red = part + kMergeParts * DIMS;
+    const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6, lane = tid & 63;
+    const int VD = p.value, nb = score_blocks(positions), nmax = score_blocks(p.max_context);
+    const float2 *st = block_stats_of(p) + static_cast<size_t>(h) * nmax;
+    const int dl = tid % DIMS, q = tid / DIMS, d = min(d0 + dl, VD - 1);
+    const float *base = p.split + static_cast<size_t>(h) * nmax * VD + d;
+    const float gate = p.q[static_cast<size_t>(h) * 2 * p.head + p.head + d];
+    float mx = -__builtin_inff();
+    for (int b = tid; b < nb; b += ea::kThreads) mx = fmaxf(mx, st[b].x);
+    mx = wave_max(mx);
+    if (lane == 0) red[wave] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    float zp = 0.0f, o[kSums];
+#pragma unroll
+    for (int k = 0; k < kSums; ++k) o[k] = 0.0f;
+    for (int t0 = 0; t0 < nb; t0 += kMergeTile) {
+        const int cnt = min(kMergeTile, nb - t0);
+        for (int b = tid; b < cnt; b += ea::kThreads) {
+            const float2 s2 = st[t0 + b];
+            const float fb = expf_libm(s2.x - mx);
+            f[b] = fb;
+            zp = __builtin_fmaf(s2.y, fb, zp);
+        }
+        __syncthreads();
+        for (int b0 = q * kSums; b0 < cnt; b0 += kAhead * kMergeParts) {
+            float x[kAhead][kSums];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+                for (int k = 0; k < kSums; ++k)
+                    x[u][k] = base[static_cast<size_t>(t0 + min(b0 + u * kMergeParts + k, cnt - 1)) * VD];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u)
+#pragma unroll
+                for (int k = 0; k < kSums; ++k)
+                    if (b0 + u * kMergeParts + k < cnt) o[k] = __builtin_fmaf(x[u][k], f[b0 + u * kMergeParts + k], o[k]);
+        }
+        __syncthreads();
+    }
+    zp = wave_sum(zp);
+    if (lane == 0) red[wave] = zp;
+#pragma unroll
+    for (int k = 0; k < kSums; ++k) part[(q * kSums + k) * DIMS + dl] = o[k];
+    __syncthreads();
+    if (tid >= DIMS || d0 + dl >= VD) return;
+    const float z = (red[0] + red[1]) + (red[2] + red[3]);
+    float sum = 0.0f;
+#pragma unroll
+    for (int k = 0; k < kMergeParts; ++k) sum += part[k * DIMS + dl];
+    const float out = (sum / z) * sigmoid_ref(gate);
+    p.out[static_cast<size_t>(h) * VD + d0 + dl] = out;
+    if constexpr (DIMS == 64)
+        if (p.out_q8l) out_quantize64(p, h, d0, out, f);
 }
 
 // e_p = expf(s_p - m) of kSeg-position segments of one head, stored for the
@@ -228,6 +424,9 @@ __global__ __launch_bounds__(ea::kThreads) void attention_softmax_kernel(const A
     const int tid = static_cast<int>(threadIdx.x), wave = tid >> 6, lane = tid & 63;
     const float *sc = p.partial + static_cast<size_t>(h) * p.max_context;
     FORTAI_ATT_MARK(21);
+    // beyond exact_max there are no e values or Z tables (contexts that never
+    // get there do not wait for the position here)
+    if (p.max_context > p.exact_max && pos >= p.exact_max) return;
     // the statistics of every 64-position score block (max m_b, sum of
     // exp(s - m_b)) written by the scores kernel: one block per thread and
     // register up to kStatRegs * 256 blocks (clamped in bounds; those past the
@@ -244,7 +443,6 @@ __global__ __launch_bounds__(ea::kThreads) void attention_softmax_kernel(const A
     mt.load();  // visible after the barrier of the max below
     if (pos < 0 || pos >= p.max_context) return;
     const int n = pos + 1;
-    if (n > p.exact_max) return;  // the split-K kernels cover this position
     if (k0 * ea::kSeg >= n) return;
     const int nb = score_blocks(n);
     // m = max over every score = max over the blocks' maxima (any order and
@@ -393,6 +591,10 @@ __global__ __launch_bounds__(ea::kThreads) void attention_output_kernel(const At
     const float *ev = evals_of(p) + static_cast<size_t>(h) * p.max_context;
     const float *tab = head_tab(p, h);
     const int rows = z_lds_segments(cap);
+    if (p.max_context > p.exact_max && pos >= p.exact_max) {
+        if (pos < p.max_context) merge_block<ea::kDims>(p, h, d0, pos + 1, lds);
+        return;
+    }
     ea::ValuePieces v;
     float e4[ea::kPieces];
     int32_t tr[kTabRegs];  // walk word tid of segment r
@@ -410,7 +612,6 @@ __global__ __launch_bounds__(ea::kThreads) void attention_output_kernel(const At
     FORTAI_ATT_MARK(3);
     if (pos < 0 || pos >= p.max_context) return;
     const int positions = pos + 1;
-    if (positions > p.exact_max) return;  // the split-K kernels cover this position
     float *work = lds;
     int32_t *walk_lds = reinterpret_cast<int32_t *>(lds + ea::work_floats());
     const int nseg = ea::z_segments(positions);
@@ -438,6 +639,7 @@ __global__ __launch_bounds__(ea::kThreads) void attention_output_kernel(const At
     FORTAI_ATT_MARK(4);
 }
 
+static_assert(kMergeTile + kMergeParts * ea::kDims + 4 <= ea::work_floats(), "merge_block fits the output step's LDS");
 size_t output_lds_bytes(int positions) {
     return (ea::work_floats() + static_cast<size_t>(z_lds_segments(positions)) * ea::kZCand) * sizeof(float);
 }
@@ -475,6 +677,7 @@ static_assert(kWideDims * kWidePitchT * 2 >= kZLdsSegments * ea::kZCand * 4, "th
 
 // dynamic LDS of attention_output_wide_kernel: the transposed tile, then w of the tile
 constexpr size_t kWideLdsBytes = static_cast<size_t>(kWideDims) * kWidePitchT * 2 + kWideTile * 4;
+static_assert((kMergeTile + kMergeParts * kWideDims + 4) * sizeof(float) <= kWideLdsBytes, "merge_block fits");
 
 // halves k of dwords a (low half of the result) and b (high half)
 __device__ __forceinline__ uint32_t pick_halves(uint32_t a, uint32_t b, int hi) {
@@ -619,10 +822,13 @@ __global__ __launch_bounds__(ea::kThreads) void attention_output_wide_kernel(con
     const int pos = *p.position;
     if (pos < 0 || pos >= p.max_context) return;
     const int n = pos + 1;
-    if (n > p.exact_max) return;  // the split-K kernels cover this position
     const int slices = (p.value + kWideDims - 1) / kWideDims;
     const int h = static_cast<int>(blockIdx.x) / slices, d0 = (static_cast<int>(blockIdx.x) % slices) * kWideDims;
     const int kvh = h / (p.heads / p.kv_heads);
+    if (n > p.exact_max) {
+        merge_block<kWideDims>(p, h, d0, n, wide_lds);
+        return;
+    }
     uint16_t *vt = reinterpret_cast<uint16_t *>(wide_lds);
     float *wt = wide_lds + kWideDims * kWidePitchT / 2;
     if (p.cache_flags[kvh] == 0)
@@ -631,223 +837,13 @@ __global__ __launch_bounds__(ea::kThreads) void attention_output_wide_kernel(con
         attend_wide<false>(p, h, d0, n, vt, wt, red);
 }
 
-
-// ---------------------------------------------------------------- split-K
-// Beyond exact_max positions: each workgroup takes one kv head and a chunk of
-// kChunk positions for the whole GQA group: the chunk's max m_c, Z_c =
-// sum exp(s - m_c) and o_c = sum exp(s - m_c) v, which the merge kernel
-// combines per head: M = max m_c, Z = sum Z_c e^(m_c - M),
-// out = (sum o_c e^(m_c - M)) / Z * sigmoid(gate) (flash-decoding).  The
-// scores are the scores kernel's (the reference's per-position dots).
-
-__device__ __forceinline__ float block_max256(float v, float *red) {
-    v = wave_max(v);
-    const int tid = static_cast<int>(threadIdx.x);
-    __syncthreads();
-    if ((tid & 63) == 0) red[tid >> 6] = v;
-    __syncthreads();
-    return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
-}
-
-__device__ __forceinline__ float block_sum256(float v, float *red) {
-    v = wave_sum(v);
-    const int tid = static_cast<int>(threadIdx.x);
-    __syncthreads();
-    if ((tid & 63) == 0) red[tid >> 6] = v;
-    __syncthreads();
-    return (red[0] + red[1]) + (red[2] + red[3]);
-}
-
-// Per-workgroup split-K partials of one kv head and chunk for the GQA group.
-// Thread t takes the 8-dim value slice t % 32 of positions t / 32 + 8 i (all
-// 32 of its 16-byte value loads in flight at once), then the 8 position
-// groups are summed through LDS.
-constexpr int kSplitSlices = 32;                    // 8-dim slices: value dims <= 256
-constexpr int kSplitGroups = 256 / kSplitSlices;    // position groups
-constexpr int kSplitPer = kChunk / kSplitGroups;    // positions per thread
-static_assert(kChunk <= 256 && kChunk % kSplitGroups == 0, "one score per thread; whole position groups");
-
-struct SplitLds {
-    float e[kMaxGroup][kChunk];
-    float red4[kMaxGroup][4];
-    float part[kMaxGroup][kSplitGroups][kSplitSlices * 8];
-};
-
-template <bool FINITE>
-__device__ __forceinline__ void split_chunk(const AttentionParams &p, int kvh, int c, int nmax, int p0, int n,
-    SplitLds &L) {
-    const int tid = static_cast<int>(threadIdx.x);
-    const int group = p.heads / p.kv_heads, VD = p.value, NKV = p.kv_heads;
-    const int slice = tid % kSplitSlices, pg = tid / kSplitSlices;
-    // the scores of every head, then the value loads (the in-order wait for
-    // the scores then does not include the values)
-    float sc[kMaxGroup], m[kMaxGroup], z[kMaxGroup];
-#pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g)
-        sc[g] = g < group ? p.partial[static_cast<size_t>(kvh * group + g) * p.max_context + p0 + min(tid, n - 1)]
-                          : 0.0f;
-    // slices past VD re-read slice 0
-    const int d0 = (slice * 8 < VD ? slice : 0) * 8;
-    const uint16_t *vb = p.vcache + (static_cast<size_t>(p0) * NKV + kvh) * VD + d0;
-    const size_t vs = static_cast<size_t>(NKV) * VD;
-    uint4 vv[kSplitPer];
-#pragma unroll
-    for (int i = 0; i < kSplitPer; ++i)
-        vv[i] = *reinterpret_cast<const uint4 *>(vb + static_cast<size_t>(min(pg + kSplitGroups * i, n - 1)) * vs);
-    FORTAI_ATT_MARK(12);
-    // the four heads' max and sum, reduced together
-#pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g) {
-        m[g] = tid < n ? sc[g] : -__builtin_inff();
-        m[g] = wave_max(m[g]);
-    }
-    if ((tid & 63) == 0)
-#pragma unroll
-        for (int g = 0; g < kMaxGroup; ++g) L.red4[g][tid >> 6] = m[g];
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g) {
-        m[g] = fmaxf(fmaxf(L.red4[g][0], L.red4[g][1]), fmaxf(L.red4[g][2], L.red4[g][3]));
-        const float ev = (g < group && tid < n) ? expf_libm(sc[g] - m[g]) : 0.0f;
-        if (tid < kChunk) L.e[g][tid] = ev;
-        z[g] = ev;
-        z[g] = wave_sum(z[g]);
-    }
-    __syncthreads();  // every wave has read red4
-    if ((tid & 63) == 0)
-#pragma unroll
-        for (int g = 0; g < kMaxGroup; ++g) L.red4[g][tid >> 6] = z[g];
-    __syncthreads();
-#pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g) z[g] = (L.red4[g][0] + L.red4[g][1]) + (L.red4[g][2] + L.red4[g][3]);
-    FORTAI_ATT_MARK(13);
-    float acc[kMaxGroup][8];
-#pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g)
-#pragma unroll
-        for (int d = 0; d < 8; ++d) acc[g][d] = 0.0f;
-#pragma unroll
-    for (int i = 0; i < kSplitPer; ++i) {
-        const int j = pg + kSplitGroups * i;
-        if (j >= n) continue;
-        const uint32_t hw[4] = {vv[i].x, vv[i].y, vv[i].z, vv[i].w};
-        float v8[8];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            v8[2 * q] = ea::kv<FINITE>(static_cast<uint16_t>(hw[q] & 0xffffu));
-            v8[2 * q + 1] = ea::kv<FINITE>(static_cast<uint16_t>(hw[q] >> 16));
-        }
-#pragma unroll
-        for (int g = 0; g < kMaxGroup; ++g) {
-            if (g >= group) break;
-            const float ej = L.e[g][j];
-#pragma unroll
-            for (int d = 0; d < 8; ++d) acc[g][d] = __builtin_fmaf(ej, v8[d], acc[g][d]);
-        }
-    }
-#pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g) {
-        if (g >= group) break;
-#pragma unroll
-        for (int d = 0; d < 8; ++d) L.part[g][pg][slice * 8 + d] = acc[g][d];
-    }
-    __syncthreads();
-    FORTAI_ATT_MARK(14);
-    if (tid >= VD) return;
-#pragma unroll
-    for (int g = 0; g < kMaxGroup; ++g) {
-        if (g >= group) break;
-        float o = 0.0f;
-#pragma unroll
-        for (int k = 0; k < kSplitGroups; ++k) o += L.part[g][k][tid];
-        float *dst = p.split + (static_cast<size_t>(kvh * group + g) * nmax + c) * (VD + 2);
-        dst[tid] = o;
-        if (tid == 0) {
-            dst[VD] = m[g];
-            dst[VD + 1] = z[g];
-        }
-    }
-}
-
-__global__ __launch_bounds__(ea::kThreads) void attention_split_kernel(const AttentionParams p_batch) {
-    const AttentionParams p = attention_seq(p_batch, static_cast<int>(blockIdx.y));
-    __shared__ SplitLds L;
-    const int pos = *p.position;
-    if (pos < 0 || pos >= p.max_context) return;
-    const int positions = pos + 1;
-    if (positions <= p.exact_max) return;  // the exact kernel covers this position
-    const int nmax = (p.max_context + kChunk - 1) / kChunk;
-    // chunk-major, like the scores kernel: chunks holding positions dispatch first
-    const int kvh = static_cast<int>(blockIdx.x) % p.kv_heads, c = static_cast<int>(blockIdx.x) / p.kv_heads;
-    const int p0 = c * kChunk;
-    if (p0 >= positions) return;
-    const int n = min(kChunk, positions - p0);
-    if (p.cache_flags[kvh] == 0) split_chunk<true>(p, kvh, c, nmax, p0, n, L);
-    else split_chunk<false>(p, kvh, c, nmax, p0, n, L);
-}
-
-// Per head and 64 value dims: the chunks' scale factors e^(m_c - M) once into
-// LDS, then each dim's chunk partials summed by four threads (a quarter of the
-// chunks each, 32 loads in flight) and combined through LDS.
-constexpr int kMaxSplitChunks = 4096;  // contexts up to 1M positions
-constexpr int kMergeDims = 64;
-constexpr int kMergeParts = ea::kThreads / kMergeDims;
-constexpr int kMergeBatch = 32;
-
-__global__ __launch_bounds__(ea::kThreads) void attention_merge_kernel(const AttentionParams p_batch) {
-    const AttentionParams p = attention_seq(p_batch, static_cast<int>(blockIdx.y));
-    __shared__ float f[kMaxSplitChunks];
-    __shared__ float red[4];
-    __shared__ float part[kMergeParts][kMergeDims];
-    const int pos = *p.position;
-    if (pos < 0 || pos >= p.max_context) return;
-    const int positions = pos + 1;
-    if (positions <= p.exact_max) return;
-    const int tid = static_cast<int>(threadIdx.x);
-    const int VD = p.value, HD = p.head;
-    const int slices = (VD + kMergeDims - 1) / kMergeDims;
-    const int h = static_cast<int>(blockIdx.x) / slices, d0 = (static_cast<int>(blockIdx.x) % slices) * kMergeDims;
-    const int nmax = (p.max_context + kChunk - 1) / kChunk, chunks = (positions + kChunk - 1) / kChunk;
-    const float *base = p.split + static_cast<size_t>(h) * nmax * (VD + 2);
-    float mx = -__builtin_inff();
-    for (int c = tid; c < chunks; c += ea::kThreads) mx = fmaxf(mx, base[static_cast<size_t>(c) * (VD + 2) + VD]);
-    mx = block_max256(mx, red);
-    float zp = 0.0f;
-    for (int c = tid; c < chunks; c += ea::kThreads) {
-        const float *row = base + static_cast<size_t>(c) * (VD + 2);
-        const float fc = expf_libm(row[VD] - mx);
-        f[c] = fc;
-        zp = __builtin_fmaf(row[VD + 1], fc, zp);
-    }
-    const float z = block_sum256(zp, red);  // (its barriers also publish f)
-    const int dl = tid % kMergeDims, q = tid / kMergeDims, d = min(d0 + dl, VD - 1);
-    const int per = (chunks + kMergeParts - 1) / kMergeParts, c0 = q * per, c1 = min(chunks, c0 + per);
-    float o = 0.0f;
-    for (int cb = c0; cb < c1; cb += kMergeBatch) {
-        float x[kMergeBatch];
-#pragma unroll
-        for (int u = 0; u < kMergeBatch; ++u) x[u] = base[static_cast<size_t>(min(cb + u, c1 - 1)) * (VD + 2) + d];
-#pragma unroll
-        for (int u = 0; u < kMergeBatch; ++u)
-            if (cb + u < c1) o = __builtin_fmaf(x[u], f[cb + u], o);
-    }
-    part[q][dl] = o;
-    __syncthreads();
-    if (q != 0 || d0 + dl >= VD) return;
-    float sum = 0.0f;
-#pragma unroll
-    for (int k = 0; k < kMergeParts; ++k) sum += part[k][dl];
-    const float gate = p.q[static_cast<size_t>(h) * 2 * HD + HD + d0 + dl];
-    const float out = (sum / z) * sigmoid_ref(gate);
-    p.out[static_cast<size_t>(h) * VD + d0 + dl] = out;
-    if (p.out_q8l) out_quantize64(p, h, d0, out, &part[1][0]);  // (wave 0 has read part)
-}
-
 }  // namespace
 
 size_t attention_scores_floats(int heads, int max_context) { return workspace_floats(heads, max_context); }
 
-int attention_split_chunks(int max_context) { return (max_context + kChunk - 1) / kChunk; }
+size_t attention_split_floats(int heads, int max_context, int value) {
+    return static_cast<size_t>(heads) * score_blocks(max_context) * value;
+}
 
 // workgroups per head of attention_softmax_kernel: one per segment for a
 // single sequence, at most 8 (each looping over segments) for a batch
@@ -874,14 +870,16 @@ hipError_t launch_attention(const AttentionParams &params, hipStream_t stream, i
     p.div_segs = fast_div(static_cast<uint32_t>(p.head / 8));
     p.div_slices = fast_div(static_cast<uint32_t>(p.value / ea::kDims));
     p.div_vd64 = fast_div(static_cast<uint32_t>(p.value / 64));
-    if (p.max_context > p.exact_max && (!p.split || attention_split_chunks(p.max_context) > kMaxSplitChunks))
-        return hipErrorInvalidValue;
+    const bool beyond = p.max_context > p.exact_max;  // (each kernel picks its regime from the device position)
+    if (beyond && (!p.split || p.max_context > kMaxSplitPositions)) return hipErrorInvalidValue;
     if (group < 1 || group > kMaxGroup || p.heads % p.kv_heads || p.head > kMaxHead || p.head % 8 ||
         p.value % ea::kDims || p.value > p.head || p.rope_dim > p.head || p.rope_dim % 2 || !p.out || !p.partial)
         return hipErrorInvalidValue;
     const int exact_positions = p.max_context < p.exact_max ? p.max_context : p.exact_max;
     const int nblk_max = (p.max_context + ea::kPosBlock - 1) / ea::kPosBlock;
-    hipLaunchKernelGGL(attention_scores_kernel, dim3(p.kv_heads * nblk_max, batch), dim3(ea::kThreads), 0, stream, p);
+    const char *first = beyond ? "attention_split_kernel" : "attention_scores_kernel";
+    hipLaunchKernelGGL(beyond ? attention_split_kernel : attention_scores_kernel, dim3(p.kv_heads * nblk_max, batch),
+        dim3(ea::kThreads), 0, stream, p);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (exact_positions > 0) {
@@ -896,29 +894,18 @@ hipError_t launch_attention(const AttentionParams &params, hipStream_t stream, i
         const int wgrid = p.heads * ((p.value + kWideDims - 1) / kWideDims);
         hipLaunchKernelGGL(attention_output_wide_kernel, dim3(wgrid, batch), dim3(ea::kThreads), wlds, stream, p);
         e = hipGetLastError();
-        note_launch("attention_scores_kernel grid %dx%d + attention_softmax_kernel grid %dx%d + "
-            "attention_output_wide_kernel grid %dx%d", p.kv_heads * nblk_max, batch,
+        note_launch("%s grid %dx%d + attention_softmax_kernel grid %dx%d + "
+            "attention_output_wide_kernel grid %dx%d", first, p.kv_heads * nblk_max, batch,
             p.heads * softmax_groups(exact_positions, batch), batch, wgrid, batch);
     } else {
         hipLaunchKernelGGL(attention_output_kernel, dim3(p.heads * (p.value / ea::kDims), batch), dim3(ea::kThreads),
             output_lds_bytes(exact_positions), stream, p);
         e = hipGetLastError();
-        note_launch("attention_scores_kernel grid %dx%d + attention_softmax_kernel grid %dx%d + "
-            "attention_output_kernel grid %dx%d", p.kv_heads * nblk_max, batch,
+        note_launch("%s grid %dx%d + attention_softmax_kernel grid %dx%d + "
+            "attention_output_kernel grid %dx%d", first, p.kv_heads * nblk_max, batch,
             p.heads * softmax_groups(exact_positions, batch), batch, p.heads * (p.value / ea::kDims), batch);
     }
-    if (e != hipSuccess || p.max_context <= p.exact_max) return e;
-    // long contexts: the split-K pair (each kernel picks its regime from the device position)
-    hipLaunchKernelGGL(attention_split_kernel, dim3(p.kv_heads * attention_split_chunks(p.max_context), batch),
-        dim3(ea::kThreads), 0, stream, p);
-    e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    hipLaunchKernelGGL(attention_merge_kernel, dim3(p.heads * ((p.value + kMergeDims - 1) / kMergeDims), batch),
-        dim3(ea::kThreads), 0, stream, p);
-    note_launch("attention_scores_kernel + attention_softmax_kernel + attention_output_kernel (positions <= %d) + "
-        "attention_split_kernel grid "
-        "%dx%d + attention_merge_kernel (beyond)", p.exact_max, p.kv_heads * attention_split_chunks(p.max_context), batch);
-    return hipGetLastError();
+    return e;
 }
 
 }  // namespace fortai_hip

@@ -1470,7 +1470,7 @@ int fortai_hip_qwen35_attention_create(fortai_hip_q8_context *c, const fortai_hi
     // changes it.
     A->exact_max = kDefaultExactMax;
     if (e == hipSuccess && max_context > A->exact_max)
-        e = alloc(&A->split, static_cast<size_t>(heads) * attention_split_chunks(max_context) * (value_size + 2));
+        e = alloc(&A->split, attention_split_floats(heads, max_context, value_size));
     if (e == hipSuccess) e = alloc(&A->cache_flags, kv_heads);
     if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
@@ -2139,7 +2139,7 @@ int fortai_hip_qwen35_batch_create(fortai_hip_q8_context *c, int batch, int laye
             if (e == hipSuccess) e = alloc(&L.attn_out, B * A->heads * A->value);
             if (e == hipSuccess) e = alloc(&L.flags, B * A->kv_heads);
             if (e == hipSuccess && max_context > A->exact_max)
-                e = alloc(&L.split, B * A->heads * attention_split_chunks(max_context) * (A->value + 2));
+                e = alloc(&L.split, B * attention_split_floats(A->heads, max_context, A->value));
         }
     }
     if (e == hipSuccess) e = upload_f32(&b->output_norm, output_norm, hidden, c->stream);
@@ -2484,7 +2484,7 @@ int fortai_hip_qwen35_attention_set_exact_max(fortai_hip_qwen35_attention *A, in
     (void)hipSetDevice(c->device);
     hipError_t e = hipSuccess;
     if (A->max_context > exact_max && !A->split)
-        e = alloc(&A->split, static_cast<size_t>(A->heads) * attention_split_chunks(A->max_context) * (A->value + 2));
+        e = alloc(&A->split, attention_split_floats(A->heads, A->max_context, A->value));
     if (e == hipSuccess) A->exact_max = exact_max;
     return done(c, e, "Qwen attention exact_max");
 }

@@ -240,30 +240,30 @@ struct AttentionParams {
     int *cache_flags = nullptr;     // [kv_heads]: 1 once the cache holds an exponent-31 half
     float *out = nullptr;           // [heads][value] gated output
     // optional (batches): the same output also as the Q8L activation of the o
-    // projection, [batch][q8l_bytes(heads * value)], written by the wide and
-    // merge kernels (value % 64 == 0 and heads * value % 128 == 0)
+    // projection, [batch][q8l_bytes(heads * value)], written by the wide
+    // kernel (value % 64 == 0 and heads * value % 128 == 0)
     void *out_q8l = nullptr;
     const int *position = nullptr;  // device position (the new token's index)
     int heads = 0, kv_heads = 0, head = 0, value = 0, max_context = 0, rope_dim = 0;
     float eps = 0.0f;
     // Up to exact_max positions the output is the reference's two-pass softmax
-    // with its summation orders (bit-exact); beyond, split-K over chunks of
+    // with its summation orders (bit-exact); beyond, split-K over blocks of
     // the context with an online-softmax merge (within 1e-3 relative).  The
-    // split-K kernels are launched only when max_context > exact_max.
+    // split-K kernel is launched only when max_context > exact_max.
     int exact_max = 1 << 30;
-    float *split = nullptr;         // [heads][attention_split_chunks][value + 2]
+    float *split = nullptr;         // [heads][64-position blocks][value] (attention_split_floats)
     int z_skew = 0;                 // test hook: offset of the Z candidate windows (0 in use)
     int force_wide = 0;             // test hook: the batches' wide output kernel for one sequence too
     // the kernels' divisors, set by launch_attention from the fields above:
     // heads, kv_heads, heads / kv_heads, head, head / 8, value / 8, value / 64
     FastDiv div_heads, div_kv_heads, div_group, div_head, div_segs, div_slices, div_vd64;
 };
-int attention_split_chunks(int max_context);
+size_t attention_split_floats(int heads, int max_context, int value);
 // batch > 1: sequences along blockIdx.y, every buffer [batch][single size],
 // position[batch]
 hipError_t launch_attention(const AttentionParams &p, hipStream_t stream, int batch = 1);
 // whether launch_attention honours p.out_q8l for this shape and batch (the
-// wide output kernel and the split-K merge write it)
+// wide output kernel writes it)
 bool attention_quantizes_output(const AttentionParams &p, int batch);
 size_t attention_scores_floats(int heads, int max_context);
 

@@ -373,6 +373,61 @@ def test_attention_output_kernels(ctx, oracle, L, wide, big):
             w.free()
 
 
+@pytest.mark.parametrize("L,heads,kvh,head", [(1, 4, 2, 64), (63, 3, 1, 64), (64, 4, 4, 128), (65, 4, 2, 64),
+                                              (2049, 4, 1, 256), (65601, 4, 2, 64)])
+def test_attention_beyond_exact_limit(ctx, oracle, L, heads, kvh, head):
+    """The split path at every position (exact_max 0): partial and whole 64-position blocks, one to four
+    heads per kv head, and more blocks than one merge tile (1024).  Against the softmax in 64 bits on the
+    oracle's q and caches: a score is a sequential fp32 dot, off by at most ds = head u sum|q k| / sqrt(head),
+    a weight by 2 ds, expf, the block factors and Z by a few u, and the sums (8 positions, 8 groups, up to
+    65 blocks and 32 parts, left to right) by 113 u; 200 u covers those, all times sum w|v|.  The
+    per-slice and the wide output kernel merge in the same order, so they agree bit for bit."""
+    rng = np.random.default_rng(L + heads)
+    mk = lambda rows, width: B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    ws = [mk(heads * 2 * head, 32), mk(kvh * head, 32), mk(kvh * head, 32), mk(32, heads * head)]
+    qn = (1 + 0.05 * rng.standard_normal(head)).astype(np.float32)
+    kn = (1 + 0.05 * rng.standard_normal(head)).astype(np.float32)
+    maxc = max(L, 64)
+    kc, vc = np.zeros(maxc * kvh * head, np.uint16), np.zeros(maxc * kvh * head, np.uint16)
+    n = (L - 1) * kvh * head
+    kc[:n] = rng.standard_normal(n).astype(np.float16).view(np.uint16)
+    vc[:n] = rng.standard_normal(n).astype(np.float16).view(np.uint16)
+    q = rng.standard_normal(heads * 2 * head).astype(np.float32)
+    k, v = (rng.standard_normal(kvh * head).astype(np.float32) for _ in range(2))
+    outs = []
+    for wide in (False, True):
+        A = B.Attention(ctx, *ws, qn, kn, heads, kvh, head, head, maxc, 64, 1.0e7, 1e-6)
+        A.set_exact_max(0)
+        A.set_test_options(force_wide=wide)
+        A.set_cache(kc, vc, maxc)
+        ctx.set_position(L - 1)
+        bufs = [ctx.upload_array(q), ctx.upload_array(k), ctx.upload_array(v), ctx.alloc(heads * head * 4)]
+        ctx.call("fortai_hip_qwen35_attention_core_device", A.h, *(b.ptr for b in bufs))
+        outs.append(bufs[3].download(np.float32))
+        for x in (*bufs, A):
+            x.free()
+    for w in ws:
+        w.free()
+    qw, kw, scores, ref = q.copy(), k.copy(), np.zeros(maxc, np.float32), np.zeros(heads * head, np.float32)
+    oracle.attention_core_step(qw, kw, v, qn, kn, kc, vc, heads, kvh, head, head, L - 1, 64, np.float32(1e7),
+                               np.float32(1e-6), scores, ref)
+    u = 2.0 ** -24
+    K = kc.view(np.float16).reshape(maxc, kvh, head)[:L].astype(np.float64)
+    V = vc.view(np.float16).reshape(maxc, kvh, head)[:L].astype(np.float64)
+    Q = qw.reshape(heads, 2, head).astype(np.float64)
+    for h in range(heads):
+        kh, vh, qh = K[:, h * kvh // heads], V[:, h * kvh // heads], Q[h, 0]
+        sc = kh @ qh / np.sqrt(head)
+        w = np.exp(sc - sc.max())
+        w /= w.sum()
+        want = (w @ vh) / (1.0 + np.exp(-Q[h, 1]))
+        ds = head * u * (np.abs(kh) @ np.abs(qh)).max() / np.sqrt(head)
+        bound = (2 * ds + 200 * u) * (w @ np.abs(vh))
+        got = outs[0].reshape(heads, head)[h]
+        assert np.all(np.abs(got - want) <= bound), f"head {h}: {np.max(np.abs(got - want) / bound)} of the bound"
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+
+
 def test_f16_lm_head_and_argmax(ctx, oracle):
     rng = np.random.default_rng(3)
     rows, width = 248320, 1024
