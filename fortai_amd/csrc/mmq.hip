@@ -251,13 +251,13 @@ constexpr int kFewRows = 128, kFewTokens = 32;
 constexpr int kCus = 256;  // compute units (the launches' tile rules)
 
 template <int EPI, bool BLOCKS>
-__global__ __launch_bounds__(256, 2) void q8_mmq_few_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
+__global__ __launch_bounds__(256, 2) void q8_mmq_kernel_few(Q8Matrix w, const int8_t *__restrict__ xq,
     const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
     const float *__restrict__ resid, int token_tiles) {
     __shared__ __align__(16) float scales[4][4][kFewTokens];  // per wave: a chunk's token scales [block][token]
     const int tid = static_cast<int>(threadIdx.x), lane = tid & 63, wave = tid >> 6;
     const int i = lane & 31, h = lane >> 5;
-    // XCD-grouped as q8_mmq_exact_small_kernel's workgroups
+    // XCD-grouped as q8_mmq_exact_kernel_small's workgroups
     const int id = static_cast<int>(blockIdx.x);
     const bool grouped = w.rows > 7 * kFewRows;
     const int row_tile = grouped ? id / 8 / token_tiles * 8 + id % 8 : id / token_tiles;
@@ -565,7 +565,7 @@ constexpr int kSmallRows = 32;   // rows per workgroup: two wave pairs of 16
 constexpr int kSmallAhead = 4;   // chunks in flight (8: the same, with more registers)
 
 template <int TT, int EPI, bool BLOCKS>
-__global__ __launch_bounds__(256, 2) void q8_mmq_exact_small_kernel(Q8Matrix w, const int8_t *__restrict__ xq,
+__global__ __launch_bounds__(256, 2) void q8_mmq_exact_kernel_small(Q8Matrix w, const int8_t *__restrict__ xq,
     const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
     const float *__restrict__ resid, int token_tiles) {
     __shared__ float hand[2][TT * 16][64];
@@ -755,9 +755,9 @@ hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, fl
             auto go = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld, out, ld_out, resid, tt_n);
             };
-            if (blocks) resid ? go(q8_mmq_exact_small_kernel<TT, 1, true>) : go(q8_mmq_exact_small_kernel<TT, 0, true>);
-            else resid ? go(q8_mmq_exact_small_kernel<TT, 1, false>) : go(q8_mmq_exact_small_kernel<TT, 0, false>);
-            note_launch("q8_mmq_exact_small_kernel<%d,%s> grid %d", TT, resid ? "add" : "store", sgrid.x);
+            if (blocks) resid ? go(q8_mmq_exact_kernel_small<TT, 1, true>) : go(q8_mmq_exact_kernel_small<TT, 0, true>);
+            else resid ? go(q8_mmq_exact_kernel_small<TT, 1, false>) : go(q8_mmq_exact_kernel_small<TT, 0, false>);
+            note_launch("q8_mmq_exact_kernel_small<%d,%s> grid %d", TT, resid ? "add" : "store", sgrid.x);
         };
         if (one <= two) small(std::integral_constant<int, 1>{});
         else small(std::integral_constant<int, 2>{});
@@ -793,9 +793,9 @@ hipError_t launch_q8_mmq(const Q8Matrix &w, const void *x8, int tokens, float *o
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld, out, ld_out, resid, tt_n);
         };
-        if (layout == X8Layout::BLOCKS) resid ? go(q8_mmq_few_kernel<1, true>) : go(q8_mmq_few_kernel<0, true>);
-        else resid ? go(q8_mmq_few_kernel<1, false>) : go(q8_mmq_few_kernel<0, false>);
-        note_launch("q8_mmq_few_kernel<%s> grid %d", resid ? "add" : "store", sgrid.x);
+        if (layout == X8Layout::BLOCKS) resid ? go(q8_mmq_kernel_few<1, true>) : go(q8_mmq_kernel_few<0, true>);
+        else resid ? go(q8_mmq_kernel_few<1, false>) : go(q8_mmq_kernel_few<0, false>);
+        note_launch("q8_mmq_kernel_few<%s> grid %d", resid ? "add" : "store", sgrid.x);
         return hipGetLastError();
     }
     const dim3 grid((w.rows + kRowTile - 1) / kRowTile, ld / kTokTile);
