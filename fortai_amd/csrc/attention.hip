@@ -152,8 +152,9 @@ __device__ __forceinline__ void split_values(const AttentionParams &p, const uin
 // One block of kPosBlock positions of one kv head, for its GQA group.
 // SPLIT (beyond exact_max): instead of the scores, the block's max m_b, sum
 // Z_b of exp(s - m_b) and value sums o_b = sum exp(s - m_b) v, which merge_block
-// combines (flash-decoding).
-template <bool SPLIT>
+// combines (flash-decoding).  UNROLLED: the scores of 256-wide heads fully
+// unrolled (more registers).
+template <bool SPLIT, bool UNROLLED>
 __device__ __forceinline__ void scores_block(const AttentionParams &p, int pos, ScoresLds &L) {
     float *qh = L.qh, *kn = L.kn;
     float2 *rs = L.rs;
@@ -261,7 +262,7 @@ __device__ __forceinline__ void scores_block(const AttentionParams &p, int pos, 
         if (j < n) {
             const float *qg = qh + gi * HD;
             const uint16_t *kr = &ktile[j][0];
-            if (finite) sc = !SPLIT && HD == 256 ? ea::score_n<true, 256>(qg, kr, sqrt_head) : ea::score<true>(qg, kr, HD, sqrt_head);
+            if (finite) sc = UNROLLED && HD == 256 ? ea::score_n<true, 256>(qg, kr, sqrt_head) : ea::score<true>(qg, kr, HD, sqrt_head);
             else sc = ea::score<false>(qg, kr, HD, sqrt_head);
             if constexpr (!SPLIT) p.partial[static_cast<size_t>(kvh * group + gi) * p.max_context + p0 + j] = sc;
         }
@@ -283,16 +284,16 @@ __device__ __forceinline__ void scores_block(const AttentionParams &p, int pos, 
     if constexpr (SPLIT) {
         // the new position's values come from the projection, not from the cache
         if (owns_new) {
+            // (loaded and rounded once: inside the loop's branch each position would wait for its own loads)
             const float *vn = p.v + static_cast<size_t>(kvh) * VD + vd0;
+            uint32_t w[4];
 #pragma unroll
-            for (int i = 0; i < kSplitPer; ++i) {
-                if (p0 + vpg * kSplitPer + i < pos) continue;  // at pos, and the clamped copies of it
-                uint32_t w[4];
+            for (int d = 0; d < 4; ++d)
+                w[d] = float_to_half_kv(vn[2 * d]) | static_cast<uint32_t>(float_to_half_kv(vn[2 * d + 1])) << 16;
+            const uint4 row = make_uint4(w[0], w[1], w[2], w[3]);
 #pragma unroll
-                for (int d = 0; d < 4; ++d)
-                    w[d] = float_to_half_kv(vn[2 * d]) | static_cast<uint32_t>(float_to_half_kv(vn[2 * d + 1])) << 16;
-                vv[i] = make_uint4(w[0], w[1], w[2], w[3]);
-            }
+            for (int i = 0; i < kSplitPer; ++i)
+                if (p0 + vpg * kSplitPer + i >= pos) vv[i] = row;  // pos, and the clamped copies of it
         }
         __syncthreads();  // every wave is done with qh and the key tile
         qh[tid] = ev;     // [head][position]; 0 past n and past the group
@@ -311,7 +312,7 @@ __global__ __launch_bounds__(ea::kThreads) void attention_scores_kernel(const At
     FORTAI_ATT_MARK(16);
     const int pos = *p.position;
     if (pos < 0 || pos >= p.max_context) return;  // never index past the cache
-    scores_block<false>(p, pos, L);
+    scores_block<false, true>(p, pos, L);
 }
 
 // The first kernel of contexts longer than exact_max: the scores up to it,
@@ -322,15 +323,16 @@ __global__ __launch_bounds__(ea::kThreads) void attention_scores_kernel(const At
 // values are loaded into the keys' registers, and the scores run in the rolled
 // form (unrolled, at three waves per SIMD: 24 against 21-22 us).  A pass over
 // the scores with the values, 256 positions per workgroup, and the merge were
-// launches of their own before: 8 heads, 32768 positions, whole call 38.3 ->
-// 28.7 us (67 MB: 2.3 TB/s).
+// launches of their own before: 8 heads, whole call at 8300 positions 31.1 ->
+// 20.4 us, 20000: 33.4 -> 24.2, 32768: 38.1 -> 29.0 (67 MB: 2.3 TB/s), 65536:
+// 54.4 -> 43.6.
 __global__ __launch_bounds__(ea::kThreads, 4) void attention_split_kernel(const AttentionParams p_batch) {
     const AttentionParams p = attention_seq(p_batch, static_cast<int>(blockIdx.y));
     __shared__ __align__(16) ScoresLds L;
     const int pos = *p.position;
     if (pos < 0 || pos >= p.max_context) return;
-    if (pos + 1 > p.exact_max) scores_block<true>(p, pos, L);
-    else scores_block<false>(p, pos, L);
+    if (pos + 1 > p.exact_max) scores_block<true, false>(p, pos, L);
+    else scores_block<false, false>(p, pos, L);
 }
 
 // Beyond exact_max, DIMS value dims of head h from the blocks' partials:
