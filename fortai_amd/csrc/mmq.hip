@@ -36,8 +36,8 @@
 // so the products pair up whatever k order the instruction uses internally.
 #include "fortai_hip_internal.h"
 #include "fortai_hip_kernels.h"
+#include "mmq_tiles.h"
 
-#include <algorithm>
 #include <type_traits>
 
 
@@ -247,9 +247,6 @@ __global__ __launch_bounds__(kMmqThreads, 4) void q8_mmq_kernel(Q8Matrix w, cons
 // workgroup share the tokens.  Operands are loaded two chunks ahead.  With the
 // quantizer, 128 x 128 tiles before: 9216 x 2560, 77 tokens 57 -> 21 us;
 // 2560 x 9216, 301 tokens 192 -> 63 us; 32 x 2560, 2103 tokens 61 -> 24 us.
-constexpr int kFewRows = 128, kFewTokens = 32;
-constexpr int kCus = 256;  // compute units (the launches' tile rules)
-
 template <int EPI, bool BLOCKS>
 __global__ __launch_bounds__(256, 2) void q8_mmq_kernel_few(Q8Matrix w, const int8_t *__restrict__ xq,
     const float *__restrict__ xs, int tokens, int ld, float *__restrict__ out, int ld_out,
@@ -259,7 +256,7 @@ __global__ __launch_bounds__(256, 2) void q8_mmq_kernel_few(Q8Matrix w, const in
     const int i = lane & 31, h = lane >> 5;
     // XCD-grouped as q8_mmq_exact_kernel_small's workgroups
     const int id = static_cast<int>(blockIdx.x);
-    const bool grouped = w.rows > 7 * kFewRows;
+    const bool grouped = w.rows > 7 * kFewRows;  // few_grouped
     const int row_tile = grouped ? id / 8 / token_tiles * 8 + id % 8 : id / token_tiles;
     const int t0 = (grouped ? id / 8 % token_tiles : id % token_tiles) * kFewTokens;
     const int row = row_tile * kFewRows + 32 * wave + i;
@@ -568,8 +565,6 @@ __global__ __launch_bounds__(kXThreads, 2) void q8_mmq_exact_kernel(Q8Matrix w, 
 // 2560 x 9216, 16 tokens 151 -> 29 / 48 us; 1024 x 3584, 77 tokens 63 -> 15 /
 // 23 us; 32 x 2560, 4096 tokens 57 -> 22 / 23 us; 9216 x 2560, 33 tokens 46 -> 29 us
 // (block-major: the 64 x 64 tiles).
-constexpr int kSmallRows = 32;   // rows per workgroup: two wave pairs of 16
-
 constexpr int kSmallAhead = 4;   // chunks in flight (8: the same, with more registers)
 
 template <int TT, int EPI, bool BLOCKS>
@@ -585,7 +580,7 @@ __global__ __launch_bounds__(256, 2) void q8_mmq_exact_kernel_small(Q8Matrix w, 
     // tiles of a row tile are consecutive there, so its L2 serves them the
     // weights; fewer row tiles would leave XCDs idle that way
     const int id = static_cast<int>(blockIdx.x);
-    const bool grouped = w.rows > 7 * kSmallRows;  // (w.rows + 31) / 32 >= 8, as the launch has it
+    const bool grouped = w.rows > 7 * kSmallRows;  // few_grouped
     const int row_tile = grouped ? id / 8 / token_tiles * 8 + id % 8 : id / token_tiles;
     const int t0 = (grouped ? id / 8 % token_tiles : id % token_tiles) * (16 * TT);
     if (row_tile * kSmallRows >= w.rows) return;  // (the grid is padded to whole groups of eight)
@@ -740,26 +735,13 @@ hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, fl
     const int8_t *xq = static_cast<const int8_t *>(x8);
     const float *xs = reinterpret_cast<const float *>(xq + static_cast<size_t>(ld) * w.chunks * 4 * 32);
     const dim3 grid((w.rows + kXTile - 1) / kXTile, (tokens + kXTile - 1) / kXTile);
-    // Time per chunk (four blocks of width) by workgroups per CU, us, measured
-    // over rows 16 .. 9216, widths 1024 .. 9216 and 1 .. 1200 tokens: 64 x 64
-    // tiles 2.15 while each CU has at most one, then 3.1 for two and 1.6 for
-    // each more; 32 rows x 16 tokens 0.15 + 0.29 each, x 32 tokens 0.25 + 0.47
-    // each (a workgroup of either does 1/8 or 1/4 of the large one's work), and
-    // 0.05 + 0.85, 0.1 + 1.07 when block-major tokens crowd two L2 channels.
-    auto per_cu = [&](int row_tile, int token_tile) {
-        const long long wgs = static_cast<long long>((w.rows + row_tile - 1) / row_tile) * ((tokens + token_tile - 1) / token_tile);
-        return static_cast<double>((wgs + kCus - 1) / kCus);
-    };
-    const double nb = per_cu(kXTile, kXTile);
-    const double large = nb <= 1.0 ? 2.15 : std::max(3.1, 1.6 * nb);
     const bool blocks = layout == X8Layout::BLOCKS;
-    const double one = (blocks ? 0.05 : 0.15) + (blocks ? 0.85 : 0.29) * per_cu(kSmallRows, 16);
-    const double two = (blocks ? 0.1 : 0.25) + (blocks ? 1.07 : 0.47) * per_cu(kSmallRows, 32);
-    if (std::min(one, two) < large) {
+    const ExactTiles tiles = exact_tiles(w.rows, tokens, blocks);
+    if (tiles != ExactTiles::LARGE) {
         auto small = [&](auto tt_c) {
             constexpr int TT = decltype(tt_c)::value;
-            const int tt_n = (tokens + 16 * TT - 1) / (16 * TT), rt_n = (w.rows + kSmallRows - 1) / kSmallRows;
-            const dim3 sgrid((rt_n >= 8 ? (rt_n + 7) / 8 * 8 : rt_n) * tt_n);
+            const int tt_n = static_cast<int>(tiles_of(tokens, 16 * TT));
+            const dim3 sgrid(static_cast<unsigned>(few_grid(w.rows, tokens, kSmallRows, 16 * TT)));
             auto go = [&](auto kernel) {
                 hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld, out, ld_out, resid, tt_n);
             };
@@ -767,7 +749,7 @@ hipError_t launch_q8_mmq_exact(const Q8Matrix &w, const void *x8, int tokens, fl
             else resid ? go(q8_mmq_exact_kernel_small<TT, 1, false>) : go(q8_mmq_exact_kernel_small<TT, 0, false>);
             note_launch("q8_mmq_exact_kernel_small<%d,%s> grid %d", TT, resid ? "add" : "store", sgrid.x);
         };
-        if (one <= two) small(std::integral_constant<int, 1>{});
+        if (tiles == ExactTiles::SMALL_16) small(std::integral_constant<int, 1>{});
         else small(std::integral_constant<int, 2>{});
         return hipGetLastError();
     }
@@ -787,17 +769,9 @@ hipError_t launch_q8_mmq(const Q8Matrix &w, const void *x8, int tokens, float *o
     const int ld = q8_tokens_ld(tokens);
     const int8_t *xq = static_cast<const int8_t *>(x8);
     const float *xs = reinterpret_cast<const float *>(xq + static_cast<size_t>(ld) * w.chunks * 4 * 32);
-    // Time per chunk by workgroups per CU, us, measured as for the exact
-    // product: 128 x 128 tiles 1.75 while each CU has at most one, then 1.65
-    // each; 128 rows x 32 tokens (a quarter of the work) 0.2 + 0.66 each.
-    auto per_cu = [&](int row_tile, int token_tile) {
-        const long long wgs = static_cast<long long>((w.rows + row_tile - 1) / row_tile) * ((tokens + token_tile - 1) / token_tile);
-        return static_cast<double>((wgs + kCus - 1) / kCus);
-    };
-    const double nl = per_cu(kRowTile, kTokTile);
-    if (!dots && 0.2 + 0.66 * per_cu(kFewRows, kFewTokens) < (nl <= 1.0 ? 1.75 : 1.65 * nl)) {
-        const int tt_n = (tokens + kFewTokens - 1) / kFewTokens, rt_n = (w.rows + kFewRows - 1) / kFewRows;
-        const dim3 sgrid((rt_n >= 8 ? (rt_n + 7) / 8 * 8 : rt_n) * tt_n);
+    if (!dots && few_tiles(w.rows, tokens)) {
+        const int tt_n = static_cast<int>(tiles_of(tokens, kFewTokens));
+        const dim3 sgrid(static_cast<unsigned>(few_grid(w.rows, tokens, kFewRows, kFewTokens)));
         auto go = [&](auto kernel) {
             hipLaunchKernelGGL(kernel, sgrid, dim3(256), 0, stream, w, xq, xs, tokens, ld, out, ld_out, resid, tt_n);
         };

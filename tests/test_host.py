@@ -255,3 +255,59 @@ int main() {
     subprocess.run([gxx, "-O2", "-I", os.path.join(ROOT, "fortai_amd", "csrc"), str(src), "-o", str(exe)], check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
     assert r.returncode == 0, r.stdout
+
+
+def test_token_product_tile_rules(tmp_path):
+    """fortai_amd/csrc/mmq_tiles.h against the kernels' own mapping, counted
+    workgroup by workgroup: the grid covers every tile once, the busiest CU's
+    workgroups are those of the busiest of eight dies of 32 CUs, and the choice
+    follows that count (777 rows x 257 tokens: two 32 x 32 workgroups on some
+    CUs, so 64 x 64 tiles for block-major tokens)."""
+    import shutil
+    gxx = shutil.which("g++")
+    if gxx is None:
+        pytest.skip("g++ not available")
+    src = tmp_path / "tiles.cpp"
+    src.write_text(r'''
+#include "mmq_tiles.h"
+#include <cstdio>
+#include <vector>
+using namespace fortai_hip;
+// as q8_mmq_exact_kernel_small and q8_mmq_kernel_few number their workgroups
+static int check(int rows, int tokens, int rt, int tt) {
+    const int tn = (tokens + tt - 1) / tt, rn = (rows + rt - 1) / rt;
+    const bool grouped = rows > 7 * rt;
+    std::vector<int> seen(static_cast<size_t>(tn) * rn);
+    int die[8] = {};
+    const long long grid = few_grid(rows, tokens, rt, tt);
+    for (long long id = 0; id < grid; ++id) {
+        const long long r = grouped ? id / 8 / tn * 8 + id % 8 : id / tn, t = grouped ? id / 8 % tn : id % tn;
+        if (r * rt >= rows) continue;
+        ++seen[r * tn + t];
+        ++die[id % 8];
+    }
+    int most = 0, bad = 0;
+    for (int d : die) most = d > most ? d : most;
+    for (int n : seen) bad += n != 1;
+    return bad + (busiest_cu(rows, tokens, rt, tt, true) != (most + 31) / 32);
+}
+int main() {
+    long bad = 0;
+    const int rows[] = {1, 31, 32, 33, 223, 224, 225, 256, 257, 400, 777, 896, 897, 1024, 1030, 2560, 3584, 9216};
+    for (int r : rows)
+        for (int t = 1; t <= 1300; t += t < 70 ? 1 : 37)
+            bad += check(r, t, 32, 16) + check(r, t, 32, 32) + check(r, t, 128, 32);
+    bad += exact_tiles(777, 257, true) != ExactTiles::LARGE;
+    bad += exact_tiles(777, 256, true) != ExactTiles::SMALL_32;  // 32 workgroups on the busiest die
+    bad += exact_tiles(600, 341, true) != ExactTiles::LARGE;
+    bad += exact_tiles(768, 320, true) != ExactTiles::SMALL_32;  // 24 row tiles: three on every die
+    bad += exact_tiles(400, 257, true) != ExactTiles::SMALL_32;  // 34 of 32 x 16 on a die, 18 of 32 x 32
+    printf("%ld\n", bad);
+    return bad != 0;
+}
+''')
+    exe = tmp_path / "tiles"
+    subprocess.run([gxx, "-O2", "-std=c++17", "-I", os.path.join(ROOT, "fortai_amd", "csrc"), str(src), "-o", str(exe)],
+                   check=True)
+    r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=120)
+    assert r.returncode == 0, r.stdout
