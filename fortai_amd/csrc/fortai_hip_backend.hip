@@ -1314,16 +1314,20 @@ namespace {
 // alone as the serial chain (0.27 us per step, 2.1 us with all of it in the
 // chain), the same bits.  The extra launches pay from 8 steps on (16 heads:
 // 8 steps 22 -> 19 us, 128 steps 267 -> 55 us).  Longer calls go
-// kStepsPerPass at a time, which bounds the scratch (one pass of the 4B
-// layer: 34 MB, kept in the context; freed and grown only between calls, so a
-// capturing stream keeps the one-launch recurrence).
+// kStepsPerPass at a time.  The scratch is one such pass whatever the call's
+// length (34 MB for the 4B layer, kept in the context), so only the first call
+// of the largest layer allocates: sized by the call, lengths rising by one
+// each freed, allocated and waited for the device (9, 10 .. 199 steps, 32
+// heads: 89 us a call, now 62).
+// Allocation is no work of a graph, so a capturing stream keeps the one-launch
+// recurrence.
 constexpr int kStepsOverTokens = 8;
 constexpr int kStepsPerPass = 1024;
 
 hipError_t enqueue_core_steps(fortai_hip_qwen35_recurrent *L, const float *qkv, const float *alpha, const float *beta,
     int steps, float *out) {
     auto *c = L->context;
-    const size_t n = static_cast<size_t>(std::min(steps, kStepsPerPass));
+    const size_t n = kStepsPerPass;
     const size_t floats = n * (L->conv_size + 2 * static_cast<size_t>(L->key_heads) + 2 * static_cast<size_t>(L->value_heads));
     hipError_t e = ensure(reinterpret_cast<void **>(&c->scratch_aux), &c->scratch_aux_bytes, floats * sizeof(float));
     float *conv = c->scratch_aux, *qinv = conv + n * L->conv_size, *kinv = qinv + n * L->key_heads;

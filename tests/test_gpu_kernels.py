@@ -488,3 +488,31 @@ def test_gdn_core_steps_lengths(ctx, steps):
     layer.free()
     for w in ws:
         w.free()
+
+
+def test_gdn_core_steps_scratch_is_kept():
+    """The token kernels' scratch is that of one pass (1024 steps) from the first
+    call on: longer calls neither allocate nor free, whose wait for the device
+    every call of a rising length would pay."""
+    ctx = B.Context(0)
+    try:
+        layer, ws, conv_w, ssm_a, ssm_dt, conv = gdn_layer_for_core(ctx, np.random.default_rng(3))
+        most = 1100
+        bufs = [ctx.alloc(most * n * 4) for n in (conv, 16, 16, 16 * 128)]
+        for b in bufs[:3]:
+            b.upload(np.zeros(b.nbytes // 4, np.float32))
+        sizes = []
+        for steps in (8, 9, 100, 1024, most, 8):
+            ctx.call("fortai_hip_qwen35_recurrent_core_steps_device", layer.h, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr,
+                     steps, bufs[3].ptr)
+            sizes.append(ctx.scratch_bytes())
+        ctx.synchronize()
+        assert len(set(sizes)) == 1, sizes
+        assert sizes[0] == 1024 * (conv + 4 * 16) * 4
+        for b in bufs:
+            b.free()
+        layer.free()
+        for w in ws:
+            w.free()
+    finally:
+        ctx.close()
