@@ -155,3 +155,57 @@ def test_exact_prefill_attention_blocks(ctx, oracle, head, heads, kvh, T, big):
         A.free()
         for w in ws:
             w.free()
+
+
+# LDS holds a block's scores beside its staging (20,480 bytes at head 256 with 4
+# queries, 24,576 with 8; 18,432 / 20,480 at 128; 17,408 / 18,432 at 64): 4
+# queries while two workgroups fit 160 KB, then 8, then 4 while one fits, then
+# the kernel for longer prompts with 2 queries (150 KB), then 1.
+@pytest.mark.parametrize("head,T,big", [
+    (256, 3840, False), (256, 3841, False), (256, 4352, True), (256, 4353, False), (256, 8960, True),
+    (128, 3968, False), (128, 3969, True), (128, 4480, False), (128, 4481, False), (64, 4544, True),
+    (256, 8961, False), (256, 8965, True), (128, 9089, False), (64, 9153, True), (256, 14848, False),
+    (256, 14849, False), (64, 18113, True)])
+def test_exact_prefill_attention_long(ctx, oracle, head, T, big):
+    """Both sides of each line of the exact kernels' query-block rule, bit for
+    bit against the reference step on rows at the edges of query blocks and key
+    tiles.  The oracle's cache is the call's own, whose sampled positions the
+    oracle writes again and must leave as they are."""
+    rng = np.random.default_rng(head + T)
+    rope = 16 if head == 64 else 64
+    mk = lambda rows, width: B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    ws = [mk(2 * head, 32), mk(head, 32), mk(head, 32), mk(32, head)]
+    qn = (1 + 0.05 * rng.standard_normal(head)).astype(np.float32)
+    kn = (1 + 0.05 * rng.standard_normal(head)).astype(np.float32)
+    A = B.Attention(ctx, *ws, qn, kn, 1, 1, head, head, T, rope, 1.0e7, 1e-6)
+    q = rng.standard_normal((T, 2 * head)).astype(np.float32)
+    k = rng.standard_normal((T, head)).astype(np.float32)
+    v = rng.standard_normal((T, head)).astype(np.float32)
+    if big:
+        v[::5, : head // 2] *= np.float32(3e5)  # exponent-31 halves
+    bufs = [ctx.upload_array(a) for a in (q, k, v)] + [ctx.alloc(T * head * 4)]
+    try:
+        ctx.call("fortai_hip_qwen35_attention_prefill_core_device", A.h, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, T, 0,
+                 bufs[3].ptr)
+        got = bufs[3].download(np.float32).reshape(T, head)
+        kc, vc = (np.array(x[: T * head], np.uint16) for x in A.cache(T))
+        kc0, vc0 = kc.copy(), vc.copy()
+        scores, want = np.zeros(T, np.float32), np.zeros(head, np.float32)
+        half = T // 2 // 64 * 64
+        sample = {0, 1, 3, 4, 7, 8, 31, 32, 63, 64, half - 1, half, half + 1, T - 1} | {T - n for n in range(2, 12)}
+        diff = []
+        for t in sorted(sample):
+            oracle.attention_core_step(q[t].copy(), k[t].copy(), v[t].copy(), qn, kn, kc, vc, 1, 1, head, head, t,
+                                       rope, np.float32(1e7), np.float32(1e-6), scores, want)
+            if not same_values(got[t], want):
+                diff.append(t)
+        assert not diff, f"exact prefill attention differs from the reference step at rows {diff}"
+        assert np.array_equal(kc, kc0) and np.array_equal(vc, vc0), "appended K/V must be bit-exact"
+        assert not big or np.any((vc & 0x7c00) == 0x7c00), "the cache holds exponent-31 halves"
+        assert np.isfinite(got).all() or big
+    finally:
+        for b in bufs:
+            b.free()
+        A.free()
+        for w in ws:
+            w.free()
