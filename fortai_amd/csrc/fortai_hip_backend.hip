@@ -1351,7 +1351,9 @@ int fortai_hip_qwen35_recurrent_core_steps_device(fortai_hip_qwen35_recurrent *L
     (void)hipSetDevice(c->device);
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     hipError_t e = hipStreamIsCapturing(c->stream, &capturing);
-    if (e == hipSuccess && L->head == 128 && steps >= kStepsOverTokens && capturing == hipStreamCaptureStatusNone) {
+    // (what neither form serves, a longer conv window, is left to the one-launch recurrence to refuse)
+    if (e == hipSuccess && L->head == 128 && L->kernel <= kConvMax && steps >= kStepsOverTokens &&
+        capturing == hipStreamCaptureStatusNone) {
         e = enqueue_core_steps(L, static_cast<const float *>(qkv), static_cast<const float *>(alpha),
             static_cast<const float *>(beta), steps, static_cast<float *>(out));
         // without memory for the scratch: the one-launch recurrence below, which needs none

@@ -516,3 +516,22 @@ def test_gdn_core_steps_scratch_is_kept():
             w.free()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("steps", [1, 7, 8, 100])
+def test_gdn_core_steps_refuse_long_windows(ctx, steps):
+    """A conv window longer than the kernels hold (8 taps) is an invalid call at
+    every number of steps, refused before anything is enqueued."""
+    layer, ws, conv_w, ssm_a, ssm_dt, conv = gdn_layer_for_core(ctx, np.random.default_rng(9), kernel=9)
+    bufs = [ctx.alloc(steps * n * 4) for n in (conv, 16, 16, 16 * 128)]
+    try:
+        code = ctx.lib.fortai_hip_qwen35_recurrent_core_steps_device(
+            layer.h, bufs[0].ptr, bufs[1].ptr, bufs[2].ptr, steps, bufs[3].ptr)
+        assert code == B.INVALID
+    finally:
+        ctx.synchronize()
+        for b in bufs:
+            b.free()
+        layer.free()
+        for w in ws:
+            w.free()
