@@ -266,7 +266,9 @@ __device__ __forceinline__ void scores_block(const AttentionParams &p, int pos, 
             else sc = ea::score<false>(qg, kr, HD, sqrt_head);
             if constexpr (!SPLIT) p.partial[static_cast<size_t>(kvh * group + gi) * p.max_context + p0 + j] = sc;
         }
-        const float mb = wave_max(sc);
+        // (from the reference's first maximum -huge: a block whose every score is
+        // -infinity then weighs 0 beside the others, not NaN)
+        const float mb = fmaxf(wave_max(sc), kLowest);
         float2 *stats = block_stats_of(p) + static_cast<size_t>(kvh * group + gi) * score_blocks(p.max_context) + b;
         if constexpr (SPLIT) {
             ev = j < n ? expf_libm(sc - mb) : 0.0f;

@@ -535,3 +535,48 @@ def test_gdn_core_steps_refuse_long_windows(ctx, steps):
         layer.free()
         for w in ws:
             w.free()
+
+
+@pytest.mark.parametrize("exact_max", [None, 0])
+@pytest.mark.parametrize("blocks", [(1, 2), (0, 1), (0, 4)])
+def test_attention_blocks_of_infinite_scores(ctx, oracle, exact_max, blocks):
+    """Whole 64-position blocks whose every score overflows to -infinity
+    (exponent-31 keys, which the reference reads as +-huge) among ordinary
+    ones: their positions weigh 0, on the exact and on the split path; with no
+    ordinary position left every output is NaN (0 / 0)."""
+    rng = np.random.default_rng(17)
+    heads, kvh, head, L = 4, 1, 256, 256
+    mk = lambda rows, width: B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    ws = [mk(heads * 2 * head, 32), mk(kvh * head, 32), mk(kvh * head, 32), mk(32, heads * head)]
+    qn, kn = np.ones(head, np.float32), np.ones(head, np.float32)
+    kn[200] = 1e6
+    A = B.Attention(ctx, *ws, qn, kn, heads, kvh, head, head, L, 64, 1.0e7, 1e-6)
+    if exact_max is not None:
+        A.set_exact_max(exact_max)
+    q = rng.standard_normal((heads, 2, head)).astype(np.float32)
+    k, v = (rng.standard_normal(kvh * head).astype(np.float32) for _ in range(2))
+    q[:, 0, 200] = 8.0  # past the rotated dims: stays > 1 normalized, so times -huge it is -infinity
+    lo, hi = (64 * b for b in blocks)
+    k[200] = -1.0 if hi == L else 0.0  # the new key: exponent 31 too, or ordinary
+    kc = rng.standard_normal((L, head)).astype(np.float16).view(np.uint16)
+    vc = rng.standard_normal((L, head)).astype(np.float16).view(np.uint16)
+    kc[lo:hi, 200] = 0xfc00
+    kc, vc = kc.ravel(), vc.ravel()
+    A.set_cache(kc, vc, L)
+    ctx.set_position(L - 1)
+    bufs = [ctx.upload_array(a.ravel()) for a in (q, k, v)] + [ctx.alloc(heads * head * 4)]
+    try:
+        ctx.call("fortai_hip_qwen35_attention_core_device", A.h, *(b.ptr for b in bufs))
+        got = bufs[3].download(np.float32)
+        want, scores = np.zeros(heads * head, np.float32), np.zeros(L, np.float32)
+        oracle.attention_core_step(q.ravel().copy(), k.copy(), v, qn, kn, kc, vc, heads, kvh, head, head, L - 1, 64,
+                                   np.float32(1e7), np.float32(1e-6), scores, want)
+        assert np.isnan(want).all() == (hi - lo == L)
+        if exact_max is None:
+            assert same_values(got, want)
+        else:
+            assert np.array_equal(np.isnan(got), np.isnan(want))
+            assert np.isnan(want).all() or rel_err(got, want) <= REL
+    finally:
+        for b in (*bufs, A, *ws):
+            b.free()
