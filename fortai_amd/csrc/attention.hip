@@ -150,8 +150,8 @@ __device__ __forceinline__ void split_values(const AttentionParams &p, const uin
 }
 
 // One block of kPosBlock positions of one kv head, for its GQA group.
-// SPLIT (beyond exact_max): instead of the scores, the block's max m_b, sum
-// Z_b of exp(s - m_b) and value sums o_b = sum exp(s - m_b) v, which merge_block
+// SPLIT (beyond exact_max): instead of the scores, the block's max m_b (or, with
+// exponent-31 halves about, a little more), sum Z_b of exp(s - m_b) and value sums o_b = sum exp(s - m_b) v, which merge_block
 // combines (flash-decoding).  UNROLLED: the scores of 256-wide heads fully
 // unrolled (more registers).
 template <bool SPLIT, bool UNROLLED>
@@ -268,7 +268,12 @@ __device__ __forceinline__ void scores_block(const AttentionParams &p, int pos, 
         }
         // (from the reference's first maximum -huge: a block whose every score is
         // -infinity then weighs 0 beside the others, not NaN)
-        const float mb = fmaxf(wave_max(sc), kLowest);
+        float mb = fmaxf(wave_max(sc), kLowest);
+        // +-huge values (exponent-31 halves): with weights of up to 1 two of them
+        // overflow the block's sum, however little the block weighs beside the
+        // others.  Relative to m_b + 5 the 64 weights sum to 64 e^-5 < 1.
+        if constexpr (SPLIT)
+            if (!finite) mb += 5.0f;
         float2 *stats = block_stats_of(p) + static_cast<size_t>(kvh * group + gi) * score_blocks(p.max_context) + b;
         if constexpr (SPLIT) {
             ev = j < n ? expf_libm(sc - mb) : 0.0f;

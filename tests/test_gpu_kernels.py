@@ -580,3 +580,49 @@ def test_attention_blocks_of_infinite_scores(ctx, oracle, exact_max, blocks):
     finally:
         for b in (*bufs, A, *ws):
             b.free()
+
+
+@pytest.mark.parametrize("new", [False, True])
+def test_attention_huge_values_of_little_weight(ctx, oracle, new):
+    """Beyond exact_max, exponent-31 values (+-huge) at positions that weigh
+    almost nothing beside one of another 64-position block: their weighted sum
+    is finite in the reference and within 1e-3 of it here.  new: the new
+    position is one of them (its block is the only one to know)."""
+    rng = np.random.default_rng(23)
+    head, L = 256, 256
+    mk = lambda rows, width: B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    ws = [mk(2 * head, 32), mk(head, 32), mk(head, 32), mk(32, head)]
+    qn, kn = np.full(head, 2.0, np.float32), np.ones(head, np.float32)
+    A = B.Attention(ctx, *ws, qn, kn, 1, 1, head, head, L, 64, 1.0e7, 1e-6)
+    A.set_exact_max(0)
+    q = rng.standard_normal(2 * head).astype(np.float32)
+    k, v = (rng.standard_normal(head).astype(np.float32) for _ in range(2))
+    kc, vc = (rng.standard_normal((L, head)).astype(np.float16).view(np.uint16) for _ in range(2))
+    huge = slice(192, 255) if new else slice(64, 128)
+    if new:
+        v[:20] = 1e6
+        vc[huge, :20] = 0x7800  # 32768: large, not of exponent 31
+    else:
+        vc[huge, :20] = 0x7c00
+    step = lambda qw, scores, out: oracle.attention_core_step(
+        qw, k.copy(), v, qn, kn, kc.ravel(), vc.ravel(), 1, 1, head, head, L - 1, 64, np.float32(1e7), np.float32(1e-6),
+        scores, out)
+    qw, scores, want = q.copy(), np.zeros(L, np.float32), np.zeros(head, np.float32)
+    step(qw, scores, want)
+    # position 10's key along the normalized, rotated q: score 32, the others about +-2 each
+    kc[10] = (qw[:head] / 2).astype(np.float16).view(np.uint16)
+    before = vc.copy()
+    before[L - 1] = 0
+    A.set_cache(kc.ravel(), before.ravel(), L)
+    ctx.set_position(L - 1)
+    bufs = [ctx.upload_array(a) for a in (q, k, v)] + [ctx.alloc(head * 4)]
+    try:
+        ctx.call("fortai_hip_qwen35_attention_core_device", A.h, *(b.ptr for b in bufs))
+        got = bufs[3].download(np.float32)
+        step(q.copy(), scores, want)
+        assert np.isfinite(want).all() and (np.abs(want[:20]) > 1e18).all()
+        assert np.max(np.abs(got[:20] / want[:20] - 1)) <= REL
+        assert rel_err(got[20:], want[20:]) <= REL
+    finally:
+        for b in (*bufs, A, *ws):
+            b.free()
