@@ -427,12 +427,14 @@ __global__ __launch_bounds__(256) void qk_rope_append_kernel(float *__restrict__
 //   s_j = (q . k_j, left to right, separately rounded) / sqrt(head)
 //   m = max s_j;  e_j = expf(s_j - m);  Z = e_0 + e_1 + ... (left to right)
 //   out_d = fl(e_0/Z v_0,d) + fl(e_1/Z v_1,d) + ... (left to right) * sigmoid(gate_d)
-// One workgroup per (block of qb queries, head, sequence).  The scores of
-// the block's keys stay in LDS (qb is chosen so that they fit); keys and
-// values pass through LDS 64 positions at a time.  A query's masked keys
+// One workgroup per (block of qb = 1 or 2 queries, head, sequence): this kernel
+// serves the prompts past the tiled one below, where the scores of more than two
+// queries do not fit in LDS.  Keys and values pass through LDS 64 positions at a
+// time.  Wave w forms the scores and weights of query w.  A query's masked keys
 // (past its position) get e = +0 and weight +0: adding +0 or -0 to a running
 // sum leaves it unchanged, so every chain can run to the block's last key.
-constexpr int kXKeys = 64;  // keys per staged tile
+constexpr int kXKeys = 64;      // keys per staged tile
+constexpr int kXFallbackQ = 2;  // queries per workgroup at most
 
 template <int HEAD>
 __global__ __launch_bounds__(256) void attention_prefill_exact_kernel(const float *__restrict__ q,
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(256) void attention_prefill_exact_kernel(const floa
         const int qi = e / HEAD, d = e % HEAD;
         qs[e] = qi < nq ? q[((static_cast<size_t>(s) * T + q0 + qi) * heads + h) * 2 * HEAD + d] : 0.0f;
     }
-    // ---- scores: thread (key j = lane, query group = wave), queries wave + 4 r
+    // ---- scores: lane = key, wave = query
     for (int j0 = 0; j0 < keys; j0 += kXKeys) {
         __syncthreads();
         for (int e = tid; e < kXKeys * (HEAD / 8); e += 256) {
@@ -466,85 +468,58 @@ __global__ __launch_bounds__(256) void attention_prefill_exact_kernel(const floa
         }
         __syncthreads();
         const int j = j0 + lane;
-        for (int r0 = 0; r0 < qb; r0 += 16) {  // up to 4 queries of this wave at a time
-            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-            for (int d = 0; d < HEAD; d += 8) {
-                const uint4 k8 = *reinterpret_cast<const uint4 *>(kv + ((d / 8) * kXKeys + lane) * 8);
-                const uint32_t kw[4] = {k8.x, k8.y, k8.z, k8.w};
-                float kf[8];
+        if (wave >= qb) continue;
+        float acc = 0.0f;
+        for (int d = 0; d < HEAD; d += 8) {
+            const uint4 k8 = *reinterpret_cast<const uint4 *>(kv + ((d / 8) * kXKeys + lane) * 8);
+            const uint32_t kw[4] = {k8.x, k8.y, k8.z, k8.w};
+            const float4 qa = *reinterpret_cast<const float4 *>(qs + wave * HEAD + d);
+            const float4 qc = *reinterpret_cast<const float4 *>(qs + wave * HEAD + d + 4);
+            const float qv[8] = {qa.x, qa.y, qa.z, qa.w, qc.x, qc.y, qc.z, qc.w};
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
-                    kf[2 * u] = gguf_half_to_real(static_cast<uint16_t>(kw[u] & 0xffffu));
-                    kf[2 * u + 1] = gguf_half_to_real(static_cast<uint16_t>(kw[u] >> 16));
-                }
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int qi = r0 + wave + 4 * r;
-                    if (qi >= qb) break;
-                    const float4 qa = *reinterpret_cast<const float4 *>(qs + qi * HEAD + d);
-                    const float4 qc = *reinterpret_cast<const float4 *>(qs + qi * HEAD + d + 4);
-                    float a = acc[r];
-                    a = a + qa.x * kf[0];
-                    a = a + qa.y * kf[1];
-                    a = a + qa.z * kf[2];
-                    a = a + qa.w * kf[3];
-                    a = a + qc.x * kf[4];
-                    a = a + qc.y * kf[5];
-                    a = a + qc.z * kf[6];
-                    a = a + qc.w * kf[7];
-                    acc[r] = a;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int qi = r0 + wave + 4 * r;
-                if (qi < qb && j < keys) sc[qi * kcap + j] = acc[r] / sqrt_head;
-            }
+            for (int u = 0; u < 8; ++u)
+                acc = acc + qv[u] * gguf_half_to_real(static_cast<uint16_t>(u & 1 ? kw[u >> 1] >> 16 : kw[u >> 1] & 0xffffu));
         }
+        if (j < keys) sc[wave * kcap + j] = acc / sqrt_head;
     }
     __syncthreads();
-    // ---- softmax weights: queries wave, wave + 4, ...; lanes over keys
+    // ---- softmax weights: wave = query, lanes over keys
     constexpr float kLowest = -3.402823466e38f;  // -huge(1.0_real32)
-    for (int qi = wave; qi < nq; qi += 4) {
-        const int n = q0 + qi + 1;  // this query's keys
-        float *row = sc + qi * kcap;
+    float *row = sc + wave * kcap;
+    if (wave < nq) {
+        const int n = q0 + wave + 1;  // this query's keys
         float m = kLowest;
         for (int j = lane; j < n; j += 64) m = fmaxf(m, row[j]);
         m = wave_max(m);
         for (int j = lane; j < keys; j += 64) row[j] = j < n ? expf_libm(row[j] - m) : 0.0f;
     }
     __syncthreads();
-    // Z of each query by one lane, left to right (masked keys add +0)
-    if (lane < 4) {
-        const int qi = wave + 4 * lane;
+    // Z of the query by one lane, left to right (masked keys add +0)
+    if (lane == 0 && wave < nq) {
         float z = 0.0f;
-        if (qi < nq) {
-            const float *row = sc + qi * kcap;
-            int j = 0;
-            for (; j + 4 <= keys; j += 4) {
-                const float4 e4 = *reinterpret_cast<const float4 *>(row + j);
-                z = z + e4.x;
-                z = z + e4.y;
-                z = z + e4.z;
-                z = z + e4.w;
-            }
-            for (; j < keys; ++j) z = z + row[j];
+        int j = 0;
+        for (; j + 4 <= keys; j += 4) {
+            const float4 e4 = *reinterpret_cast<const float4 *>(row + j);
+            z = z + e4.x;
+            z = z + e4.y;
+            z = z + e4.z;
+            z = z + e4.w;
         }
-        // the weights e_j / Z (lanes of this wave finish the row below)
-        if (qi < nq) qs[qi * HEAD] = z;  // q is no longer needed: slot 0 of the row holds Z
+        for (; j < keys; ++j) z = z + row[j];
+        qs[wave * HEAD] = z;  // q is no longer needed: slot 0 of the row holds Z
     }
     __syncthreads();
-    for (int qi = wave; qi < nq; qi += 4) {
-        const float z = qs[qi * HEAD];
-        float *row = sc + qi * kcap;
+    if (wave < nq) {
+        const float z = qs[wave * HEAD];
         for (int j = lane; j < keys; j += 64) row[j] = row[j] / z;
     }
-    // ---- P.V: thread = (dim d, queries qd, qd + QS, ...)
-    constexpr int kQS = 256 / HEAD;  // query phases per dim
+    // ---- P.V: thread = (dim d, queries qd, qd + kQS)
+    constexpr int kQS = 256 / HEAD;                                  // query phases per dim
+    constexpr int kQPT = kXFallbackQ > kQS ? kXFallbackQ / kQS : 1;  // queries per thread
     const int d = tid % HEAD, qd = tid / HEAD;
-    float acc[16];
+    float acc[kQPT];
 #pragma unroll
-    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+    for (int r = 0; r < kQPT; ++r) acc[r] = 0.0f;
     for (int j0 = 0; j0 < keys; j0 += kXKeys) {
         __syncthreads();
         for (int e = tid; e < kXKeys * (HEAD / 8); e += 256) {
@@ -560,7 +535,7 @@ __global__ __launch_bounds__(256) void attention_prefill_exact_kernel(const floa
 #pragma unroll
             for (int u = 0; u < 4; ++u) vf[u] = gguf_half_to_real(kv[min(jj + u, jn - 1) * HEAD + d]);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
+            for (int r = 0; r < kQPT; ++r) {
                 const int qi = qd + kQS * r;
                 if (qi >= nq) break;
                 const float *w = sc + qi * kcap + j0 + jj;
@@ -579,7 +554,7 @@ __global__ __launch_bounds__(256) void attention_prefill_exact_kernel(const floa
         }
     }
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
+    for (int r = 0; r < kQPT; ++r) {
         const int qi = qd + kQS * r;
         if (qi >= nq) break;
         const size_t row = (static_cast<size_t>(s) * T + q0 + qi) * heads + h;
@@ -1279,12 +1254,12 @@ hipError_t launch_attention_prefill(const AttentionParams &p, int batch, int T, 
         }
         // longer prompts: queries per workgroup so that the block's scores fit in LDS
         const int kcap4 = (T + 3) / 4 * 4;
-        int qb = 4;
+        int qb = kXFallbackQ;
         auto lds_of = [&](int b) {
             return static_cast<size_t>(b) * p.head * 4 + static_cast<size_t>(kXKeys) * p.head * 2 +
                 static_cast<size_t>(b) * kcap4 * 4;
         };
-        while (qb > 1 && lds_of(qb) > 150 * 1024) qb /= 2;
+        if (lds_of(qb) > 150 * 1024) qb = 1;
         if (lds_of(qb) > 150 * 1024) return hipErrorInvalidValue;
         const dim3 xgrid((T + qb - 1) / qb, p.heads, batch);
         switch (p.head) {
