@@ -626,3 +626,78 @@ def test_attention_huge_values_of_little_weight(ctx, oracle, new):
     finally:
         for b in (*bufs, A, *ws):
             b.free()
+
+
+@pytest.mark.parametrize("L", [1, 64, 65, 1000, 8191, 8192, 8193])
+def test_attention_exact_positions_of_long_contexts(ctx, oracle, L):
+    """A layer whose context (8300) is longer than its exact limit (8192, the
+    default) runs one first kernel for both regimes: positions up to the limit
+    bit for bit, the next one within 1e-3."""
+    rng = np.random.default_rng(L)
+    heads, kvh, head, maxc = 8, 2, 256, 8300
+    mk = lambda rows, width: B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    ws = [mk(heads * 2 * head, 32), mk(kvh * head, 32), mk(kvh * head, 32), mk(32, heads * head)]
+    qn, kn = ((1 + 0.05 * rng.standard_normal(head)).astype(np.float32) for _ in range(2))
+    A = B.Attention(ctx, *ws, qn, kn, heads, kvh, head, head, maxc, 64, 1.0e7, 1e-6)
+    kc, vc = np.zeros(maxc * kvh * head, np.uint16), np.zeros(maxc * kvh * head, np.uint16)
+    n = (L - 1) * kvh * head
+    kc[:n] = rng.standard_normal(n).astype(np.float16).view(np.uint16)
+    vc[:n] = rng.standard_normal(n).astype(np.float16).view(np.uint16)
+    A.set_cache(kc, vc, maxc)
+    q = rng.standard_normal(heads * 2 * head).astype(np.float32)
+    k, v = (rng.standard_normal(kvh * head).astype(np.float32) for _ in range(2))
+    ctx.set_position(L - 1)
+    bufs = [ctx.upload_array(a) for a in (q, k, v)] + [ctx.alloc(heads * head * 4)]
+    try:
+        ctx.call("fortai_hip_qwen35_attention_core_device", A.h, *(b.ptr for b in bufs))
+        got = bufs[3].download(np.float32)
+        want, scores = np.zeros(heads * head, np.float32), np.zeros(maxc, np.float32)
+        oracle.attention_core_step(q.copy(), k.copy(), v, qn, kn, kc, vc, heads, kvh, head, head, L - 1, 64,
+                                   np.float32(1e7), np.float32(1e-6), scores, want)
+        if L <= 8192:
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        else:
+            assert rel_err(got, want) <= REL
+        gk, gv = A.cache(L)
+        assert np.array_equal(gk, kc[:L * kvh * head]) and np.array_equal(gv, vc[:L * kvh * head])
+    finally:
+        for b in (*bufs, A, *ws):
+            b.free()
+
+
+@pytest.mark.parametrize("kernel,key_heads,value_heads", [(2, 16, 16), (3, 4, 8), (8, 16, 32), (4, 1, 3)])
+def test_gdn_core_steps_forms(ctx, kernel, key_heads, value_heads):
+    """Core steps through the token kernels for every kind of layer they take
+    (conv windows of 2 to 8 taps, grouped and odd numbers of value heads): the
+    bits of as many single core steps."""
+    rng = np.random.default_rng(kernel + key_heads)
+    head, steps, H = 128, 21, 32
+    inner = value_heads * head
+    conv = 2 * key_heads * head + inner
+    mk = lambda rows, width: B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    ws = [mk(conv, H), mk(inner, H), mk(value_heads, H), mk(value_heads, H), mk(H, inner)]
+    conv_w = (rng.standard_normal(conv * kernel) * 0.3).astype(np.float32)
+    ssm_a, ssm_dt = -rng.random(value_heads).astype(np.float32), rng.standard_normal(value_heads).astype(np.float32)
+    layer = B.Recurrent(ctx, *ws, conv_w, conv, kernel, ssm_a, ssm_dt, np.ones(head, np.float32), head, key_heads,
+                        value_heads, head, inner, 1e-6)
+    state = (rng.standard_normal(value_heads * head * head) * 0.02).astype(np.float32)
+    cstate = (rng.standard_normal((kernel - 1) * conv) * 0.5).astype(np.float32)
+    bufs = [ctx.upload_array(rng.standard_normal((steps, n)).astype(np.float32)) for n in (conv, value_heads, value_heads)]
+    bufs += [ctx.alloc(steps * inner * 4) for _ in range(2)]
+    q, a, b, one, many = bufs
+    at = lambda buf, t, n: buf.ptr.value + t * n * 4
+    bits = lambda x: np.asarray(x, np.float32).view(np.uint32)
+    try:
+        layer.set_state(state, cstate)
+        for t in range(steps):
+            ctx.call("fortai_hip_qwen35_recurrent_core_device", layer.h, at(q, t, conv), at(a, t, value_heads),
+                     at(b, t, value_heads), at(one, t, inner))
+        want, want_state = one.download(np.float32), layer.state()
+        layer.set_state(state, cstate)
+        ctx.call("fortai_hip_qwen35_recurrent_core_steps_device", layer.h, q.ptr, a.ptr, b.ptr, steps, many.ptr)
+        got, got_state = many.download(np.float32), layer.state()
+        assert np.array_equal(bits(got), bits(want))
+        assert all(np.array_equal(bits(x), bits(y)) for x, y in zip(got_state, want_state))
+    finally:
+        for x in (*bufs, layer, *ws):
+            x.free()
