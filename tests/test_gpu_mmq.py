@@ -166,6 +166,19 @@ def test_mmq_lane_order_tiles(ctx, rows, width, tokens):
     W.free()
 
 
+def fma32(a, b, c):
+    """float32 fma(a, b, c), b an integer below 2^20: the product is exact in
+    float64, and the sum is rounded to odd there (its error by TwoSum; 53 >=
+    2 x 24 + 2 bits), so that its rounding to float32 is the only one."""
+    p, c = a.astype(np.float64) * b, c.astype(np.float64)
+    s = p + c
+    bb = s - p
+    err = (p - (s - bb)) + (c - bb)
+    even = (s.view(np.uint64) & np.uint64(1)) == 0
+    odd = np.where((err != 0) & even, np.nextafter(s, np.where(err > 0, np.inf, -np.inf)), s)
+    return odd.astype(np.float32)
+
+
 @pytest.mark.parametrize("rows,width,tokens", [(1, 32, 1), (31, 96, 33), (130, 160, 64), (897, 288, 31), (1030, 1056, 40),
                                                (2560, 544, 700), (128, 2560, 129), (4100, 128, 520)])
 def test_mmq_tiles(ctx, oracle, rows, width, tokens):
@@ -192,11 +205,8 @@ def test_mmq_tiles(ctx, oracle, rows, width, tokens):
         dots = oracle.block_dots(w, qr, rows, nb).astype(np.float64)
         acc = np.zeros(rows, np.float32)
         for b in range(nb):
-            # a float64 product and sum of a 24-bit and a 20-bit factor and a
-            # float32 is exact here up to its one rounding to float32, unless
-            # the float64 sum itself rounds: allow that double rounding one ulp
-            acc = ((ws[:, b] * np.float32(sr[b])).astype(np.float64) * dots[:, b] + acc).astype(np.float32)
-        assert rel_err(got[t], acc) <= 2.0 ** -22, f"token {t}"
+            acc = fma32(ws[:, b] * np.float32(sr[b]), dots[:, b], acc)
+        assert np.array_equal(got[t].view(np.uint32), acc.view(np.uint32)), f"token {t}"
     resid = rng.standard_normal((tokens, rows)).astype(np.float32)
     out.upload(resid)
     ctx.call("fortai_hip_q8_mmq_device", ctx.h, W.h, dq.ptr, tokens, out.ptr, out.ptr, None)
