@@ -1030,6 +1030,17 @@ int fortai_hip_q8_mmq_exact_device(fortai_hip_q8_context *c, const fortai_hip_q8
     return done(c, e, "token-block matmul (lane order)");
 }
 
+int fortai_hip_q8_mmq_chunks_device(fortai_hip_q8_context *c, const fortai_hip_q8_weights *w, const void *x8, int tokens,
+    int exact, void *out, const void *resid) {
+    if (!c || !owned(c, w) || !x8 || !out || tokens <= 0) return FORTAI_HIP_INVALID;
+    (void)hipSetDevice(c->device);
+    float *o = static_cast<float *>(out);
+    const float *r = static_cast<const float *>(resid);
+    const hipError_t e = exact ? launch_q8_mmq_exact(w->m, x8, tokens, o, w->m.rows, r, X8Layout::CHUNKS, c->stream)
+                               : launch_q8_mmq(w->m, x8, tokens, o, w->m.rows, r, nullptr, X8Layout::CHUNKS, c->stream);
+    return done(c, e, "token-block matmul (chunk-major tokens)");
+}
+
 int fortai_hip_q8_mmq_block_dots(fortai_hip_q8_context *c, const fortai_hip_q8_weights *w, const void *x8,
     int tokens, void *dots) {
     if (!c || !owned(c, w) || !x8 || !dots || tokens <= 0) return FORTAI_HIP_INVALID;

@@ -665,6 +665,15 @@ FORTAI_HIP_WEAK int fortai_hip_q8_mmq_block_dots(fortai_hip_q8_context *context,
     return FORTAI_HIP_RUNTIME_ERROR;
 }
 
+FORTAI_HIP_WEAK int fortai_hip_q8_mmq_chunks_device(fortai_hip_q8_context *context,
+    const fortai_hip_q8_weights *weights, const void *device_tokens, int tokens, int exact, void *device_output,
+    const void *device_residual)
+{
+    (void)context; (void)weights; (void)device_tokens; (void)tokens; (void)exact; (void)device_output;
+    (void)device_residual;
+    return FORTAI_HIP_RUNTIME_ERROR;
+}
+
 FORTAI_HIP_WEAK int fortai_hip_qwen35_batch_create(fortai_hip_q8_context *context, int batch, int layer_count,
     fortai_hip_qwen35_recurrent *const *recurrent, fortai_hip_qwen35_attention *const *attention,
     const fortai_hip_q8_weights *const *ffn_gate, const fortai_hip_q8_weights *const *ffn_up,

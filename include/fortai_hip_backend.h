@@ -262,7 +262,12 @@ int fortai_hip_q8_batch_matvec_noalloc(fortai_hip_q8_context *context,
  * fortai_q8_dot.c:287-331): every output is bit-identical to the decode
  * matvec of its token.  The prompt prefill's default projections.
  * mmq_block_dots: the exact int32 dot of every (token, row, block), device
- * int32 [tokens][rows][width/32] (parity probe). */
+ * int32 [tokens][rows][width/32] (parity probe).
+ * mmq_chunks [test only]: either product (exact != 0: mmq_exact) over tokens in
+ * the prompt prefill's own layout, chunks of four blocks: int8
+ * [width/128 rounded up][ld][8][4][4] (values 4 l .. 4 l + 3 of block j at [l][j]),
+ * then fp32 scales [width/128 rounded up][ld][4]; ld = tokens rounded up to 128.
+ * Blocks past the width hold zeros; rows past the tokens may hold anything. */
 size_t fortai_hip_q8_tokens_bytes(int tokens, int width);
 int fortai_hip_q8_quantize_tokens_device(fortai_hip_q8_context *context,
     const void *device_x, int tokens, int width, void *device_tokens);
@@ -275,6 +280,9 @@ int fortai_hip_q8_mmq_exact_device(fortai_hip_q8_context *context,
 int fortai_hip_q8_mmq_block_dots(fortai_hip_q8_context *context,
     const fortai_hip_q8_weights *weights, const void *device_tokens, int tokens,
     void *device_dots);
+int fortai_hip_q8_mmq_chunks_device(fortai_hip_q8_context *context,
+    const fortai_hip_q8_weights *weights, const void *device_tokens, int tokens,
+    int exact, void *device_output, const void *device_residual);
 
 /* Recurrent-layer core step (conv1d + SiLU + L2 norm + decay/beta + delta
  * rule; no projections, no gated norm): device fp32 qkv [conv_size], alpha and

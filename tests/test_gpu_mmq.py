@@ -214,3 +214,40 @@ def test_mmq_tiles(ctx, oracle, rows, width, tokens):
     for b in (dx, dq, out):
         b.free()
     W.free()
+
+
+@pytest.mark.parametrize("exact", [0, 1])
+@pytest.mark.parametrize("rows,width,tokens", [(1, 32, 1), (33, 640, 17), (225, 544, 31), (264, 1664, 48), (897, 288, 31),
+                                               (1030, 1056, 40), (300, 96, 260), (2560, 544, 700), (2560, 1056, 150),
+                                               (4100, 128, 520), (2100, 96, 900)])
+def test_mmq_chunk_major_tokens(ctx, rows, width, tokens, exact):
+    """Both products over the prefill's chunk-major tokens (one and several row
+    tiles of every kind, ragged rows and tokens, whole and partial groups of
+    chunks) give the bits of the block-major ones, with and without the
+    residual, whatever the rows past the tokens hold."""
+    rng = np.random.default_rng(rows + 11 * width + tokens)
+    W = B.Q8Weights(ctx, synth.q8_blocks(rng, rows, width), rows, width)
+    dx = ctx.upload_array(rng.standard_normal((tokens, width)).astype(np.float32))
+    nbytes = B.load().fortai_hip_q8_tokens_bytes(tokens, width)
+    blocks, chunks = ctx.alloc(nbytes), ctx.alloc(nbytes)
+    want, got = ctx.alloc(tokens * rows * 4), ctx.alloc(tokens * rows * 4)
+    ctx.call("fortai_hip_q8_quantize_tokens_device", ctx.h, dx.ptr, tokens, width, blocks.ptr)
+    q, s, ld, bp = tokens_layout(ctx, blocks, tokens, width)
+    cq = q.reshape(bp // 4, 4, ld, 8, 4).transpose(0, 2, 3, 1, 4).copy()
+    cs = s.reshape(bp // 4, 4, ld).transpose(0, 2, 1).copy()
+    cq[:, tokens:], cs[:, tokens:] = -128, np.nan
+    chunks.upload(np.concatenate([cq.view(np.uint8).ravel(), cs.view(np.uint8).ravel()]))
+    entry = "fortai_hip_q8_mmq_exact_device" if exact else "fortai_hip_q8_mmq_device"
+    resid = rng.standard_normal(tokens * rows).astype(np.float32)
+    try:
+        for r in (None, resid):
+            if r is not None:
+                want.upload(r)
+                got.upload(r)
+            at = lambda b: None if r is None else b.ptr
+            ctx.call(entry, ctx.h, W.h, blocks.ptr, tokens, want.ptr, at(want), None)
+            ctx.call("fortai_hip_q8_mmq_chunks_device", ctx.h, W.h, chunks.ptr, tokens, exact, got.ptr, at(got))
+            assert np.array_equal(got.download(np.uint32), want.download(np.uint32))
+    finally:
+        for b in (dx, blocks, chunks, want, got, W):
+            b.free()
