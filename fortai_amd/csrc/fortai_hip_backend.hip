@@ -216,6 +216,12 @@ inline bool fam(unsigned f) { return (g_families & f) != 0; }
 thread_local std::vector<plan_step> *g_plan = nullptr;
 thread_local int g_plan_batch = 1;
 
+// start recording into plan, or stop (nullptr)
+void record_into(std::vector<plan_step> *plan) {
+    g_plan = plan;
+    note_launches(plan != nullptr);
+}
+
 hipError_t rec(hipError_t e, const char *operation) {
     if (e == hipSuccess && g_plan) g_plan->push_back({operation, last_launch(), g_plan_batch});
     return e;
@@ -1679,10 +1685,10 @@ hipError_t capture_decoder(fortai_hip_qwen35_decoder *d) {
     if (!d->use_graph) return hipSuccess;
     hipError_t e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
-    g_plan = &d->plan;
+    record_into(&d->plan);
     g_plan_batch = 1;
     const hipError_t ce = enqueue_decoder_step(d, c->stream);
-    g_plan = nullptr;
+    record_into(nullptr);
     e = hipStreamEndCapture(c->stream, &d->graph);
     if (ce != hipSuccess) e = ce;
     if (e == hipSuccess) e = hipGraphInstantiate(&d->exec, d->graph, nullptr, nullptr, 0);
@@ -1691,10 +1697,10 @@ hipError_t capture_decoder(fortai_hip_qwen35_decoder *d) {
 hipError_t run_step(fortai_hip_qwen35_decoder *d) {
     // the plan is recorded by the first step (at capture for the graph)
     std::vector<plan_step> *saved = g_plan;
-    if (d->plan.empty() && !d->use_graph) g_plan = &d->plan;
+    if (d->plan.empty() && !d->use_graph) record_into(&d->plan);
     const hipError_t e = d->use_graph ? hipGraphLaunch(d->exec, d->context->stream)
                                       : enqueue_decoder_step(d, d->context->stream);
-    g_plan = saved;
+    record_into(saved);
     return e;
 }
 // after a call's last step: the pending argmax finish, so token, trace and
@@ -2011,11 +2017,11 @@ hipError_t batch_step(fortai_hip_qwen35_batch *b) {
     if (b->use_graph) return hipGraphLaunch(b->exec, b->context->stream);
     std::vector<plan_step> *saved = g_plan;
     if (b->plan.empty()) {
-        g_plan = &b->plan;
+        record_into(&b->plan);
         g_plan_batch = b->batch;
     }
     const hipError_t e = enqueue_batch_step(b, b->context->stream);
-    g_plan = saved;
+    record_into(saved);
     g_plan_batch = 1;
     return e;
 }
@@ -2073,10 +2079,10 @@ hipError_t capture_batch(fortai_hip_qwen35_batch *b) {
     if (!b->use_graph) return hipSuccess;
     hipError_t e = hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return e;
-    g_plan = &b->plan;
+    record_into(&b->plan);
     g_plan_batch = b->batch;
     const hipError_t ce = enqueue_batch_step(b, c->stream);
-    g_plan = nullptr;
+    record_into(nullptr);
     g_plan_batch = 1;
     e = hipStreamEndCapture(c->stream, &b->graph);
     if (ce != hipSuccess) e = ce;
@@ -2464,10 +2470,10 @@ int fortai_hip_qwen35_batch_prefill(fortai_hip_qwen35_batch *b, const int64_t *t
     if (e == hipSuccess && kernel_ms) e = hipEventRecord(c->start, c->stream);
     const PrefillMode mode = b->prefill_mode;
     b->prefill_plan.clear();
-    g_plan = &b->prefill_plan;
+    record_into(&b->prefill_plan);
     g_plan_batch = static_cast<int>(N);
     if (e == hipSuccess) e = enqueue_batch_prefill(b, T, mode, c->stream);
-    g_plan = nullptr;
+    record_into(nullptr);
     g_plan_batch = 1;
     if (e == hipSuccess && kernel_ms) e = hipEventRecord(c->stop, c->stream);
     if (e == hipSuccess && logits)

@@ -83,8 +83,10 @@ struct MatvecInput {
     int width = 0;                // activation elements (multiple of 32)
 };
 
-// Plan recording: every launcher notes the kernel variant it launched
-// (printf-style); last_launch() returns the note of this thread's last launch.
+// Plan recording: while note_launches(true) holds for this thread, every
+// launcher notes the kernel variant it launched (printf-style); last_launch()
+// returns the note of the last launch.
+void note_launches(bool on);
 void note_launch(const char *fmt, ...);
 const char *last_launch();
 const char *prologue_name(Prologue p);
