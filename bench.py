@@ -534,11 +534,12 @@ def bench_gdn(steps: int = 128, reps: int = 8):
                                        "every step), graph replay",
                                "us_per_step": round(us, 3), "algorithmic_bytes": algo, "gbps": round(gbps, 1),
                                "frac": round(gbps / HBM_PEAK_GBPS, 4)},
-            "state_resident": {"path": "gdn_recurrence_kernel: all steps in one launch, state in registers",
+            "state_resident": {"path": "the prompt's kernels: conv1d, norms and gates of every step in parallel, then "
+                                       "gdn_prefill_kernel for the delta rule's chain, state in registers",
                                "us_per_step": round(us_res, 3), "algorithmic_bytes_per_step": int(algo_res),
                                "gbps": round(algo_res / (us_res * 1e-6) / 1e9, 1),
                                "frac": round(algo_res / (us_res * 1e-6) / 1e9 / HBM_PEAK_GBPS, 4),
-                               "note": "latency-bound: a serial chain of 128 dependent steps in 128 workgroups"}}
+                               "note": "latency-bound: a serial chain of 128 dependent steps in 256 one-wave workgroups"}}
 
 
 def bench_attention(cases=((1024, None), (4096, None), (32768, None), (32768, 1 << 20)), calls: int = 16,

@@ -20,8 +20,11 @@
 // Chunk-major, written and read inside the prompt prefill:
 //   q[(c * ld + t) * 128 + l * 16 + j * 4 + k]  int8 value 4 l + k of block 4 c + j of token t
 //   s[(c * ld + t) * 4 + j]                     its scale
-// with ld = tokens rounded up to 128 and blocks padded to a multiple of 4;
-// padding holds zeros.  The int8 part precedes the scales in one buffer of
+// with ld = tokens rounded up to 128 and blocks padded to a multiple of 4.  The
+// blocks past the width hold zeros.  Rows past the tokens are zeros too as
+// q8_quantize_tokens_kernel writes them, and undefined inside the prefill: the
+// products read them, but a token's outputs depend on its own row alone and those
+// of rows past the tokens are not stored.  The int8 part precedes the scales in one buffer of
 // q8_tokens_bytes() bytes.  Chunk-major, a token's chunk (four blocks) is 128
 // contiguous bytes, lane part by lane part as the decode layouts have it: one
 // 16-byte load gives a lane its part of four blocks, and the lines that a token

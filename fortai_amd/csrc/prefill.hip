@@ -2,14 +2,15 @@
 //
 // The reference has no prefill: it runs every prompt token through the decode
 // step (fortai_qwen35_cpu.f90:591-711).  Here the projections of all
-// batch x T tokens are token-block products on the i8 matrix cores
-// (mmq.hip), and the parts that are sequential in time run as one kernel per
-// layer that loops over the tokens: the causal conv1d (per channel,
-// :856-879), the delta rule (per value head and 16 state rows, :880-906) and
-// causal attention (per query block, online softmax).  Results agree with the
-// per-token decode within fp32 rounding (the block dots are exact; the fp32
-// accumulation orders differ), not bit for bit.  Rows are token-major: row
-// n = s * T + t is token t of sequence s, at position t.
+// batch x T tokens are token-block products on the matrix cores (mmq.hip), the
+// causal conv1d (:856-879) and the norms and gates of every token run in
+// parallel, and the delta rule (:880-906) runs over the tokens as a serial chain
+// per 8 state rows of a value head.  Causal attention (:1006-1033) runs per
+// query block.  The exact mode keeps every summation order of the per-token
+// decode (in attention the two-pass softmax) and gives its bits; the fast mode
+// (whole-block dots, fp16 matrix-core attention with an online softmax) agrees
+// with it within rounding.  Rows are token-major: row n = s * T + t is token t of
+// sequence s, at position t.
 #include "attention_exact.h"
 #include "fortai_hip_internal.h"
 #include "fortai_hip_kernels.h"
