@@ -332,7 +332,8 @@ __global__ __launch_bounds__(ea::kThreads) void attention_scores_kernel(const At
 // the scores with the values, 256 positions per workgroup, and the merge were
 // launches of their own before: 8 heads, whole call at 8300 positions 31.1 ->
 // 20.4 us, 20000: 33.4 -> 24.2, 32768: 38.1 -> 29.0 (67 MB: 2.3 TB/s), 65536:
-// 54.4 -> 43.6.
+// 54.4 -> 43.6.  Exact positions, two launches fewer behind them: 1000: 25.6 ->
+// 22.9, 4000: 32.8 -> 30.3, 8000: 43.4 -> 41.5.
 __global__ __launch_bounds__(ea::kThreads, 4) void attention_split_kernel(const AttentionParams p_batch) {
     const AttentionParams p = attention_seq(p_batch, static_cast<int>(blockIdx.y));
     __shared__ __align__(16) ScoresLds L;
